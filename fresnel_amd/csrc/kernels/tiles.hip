@@ -58,8 +58,10 @@ __device__ __forceinline__ bool tile_rect(const TileCam& c, float4 lo, float4 hi
         jmin = fminf(jmin, j_f);
         jmax = fmaxf(jmax, j_f);
         }
-    if (zmax <= 0.0f)
-        return false; // behind the camera (rays advance along -w)
+    // behind the camera (rays advance along -w), by more than the depth's and
+    // a hit distance's rounding: preview rays have tnear 0
+    if (zmax <= -0x1p-18f * sqrtf(dmax2))
+        return false;
     if (c.model == 1 && zmin <= 0.0f)
         {
         straddle = true;

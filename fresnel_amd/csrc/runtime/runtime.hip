@@ -2227,6 +2227,8 @@ static void render_path(DeviceObj& D, const std::vector<SceneObj*>& scenes, cons
         throw Error(FH_ERR_STATE, "traversal stack overflow");
     }
 
+constexpr uint32_t PREVIEW_BLOCK = 256;
+
 static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     {
     std::lock_guard<std::mutex> lock(D.mu);
@@ -2236,14 +2238,30 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     // direct tracers do not support depth of field (fresnel/cpu/TracerDirect.cc:38-40)
     fh_user_camera cam = sc.camera;
     cam.f_stop = __builtin_huge_valf();
+    update_tiles(D, sc, tr, make_cam(cam), (uint64_t)tr.W * tr.H * tr.aa_n * tr.aa_n);
     JobDev J = make_job(sc, tr, cam);
     J.K = 1;
+    set_order_divisors(J);
     tr.order_after_copies(D.stream, nullptr);
     RenderScratch& R = D.rs;
     R.jobs.ensure(1);
     HIPCHECK(hipMemcpyAsync(R.jobs.p, &J, sizeof(J), hipMemcpyHostToDevice, D.stream));
-    D.launch("preview", [&] { k_preview<<<blocks(J.npix, 64), 64, 0, D.stream>>>(R.jobs.p, tr.aa_n); });
+    // with at least as many samples as a workgroup has wavefronts they share
+    // one chunk of 64 pixels, else each takes its own
+    const bool split = (uint64_t)tr.aa_n * tr.aa_n >= PREVIEW_BLOCK / 64;
+    auto* kern = sc.sphere_leaves ? (split ? k_preview<PREVIEW_BLOCK, 8, T_SPHERES, true>
+                                           : k_preview<PREVIEW_BLOCK, 8, T_SPHERES, false>)
+                                  : (split ? k_preview<PREVIEW_BLOCK, 8, T_ALL, true>
+                                           : k_preview<PREVIEW_BLOCK, 8, T_ALL, false>);
+    const uint32_t units = blocks(blocks(J.npix, 64), split ? 1 : PREVIEW_BLOCK / 64);
+    const uint32_t grid = std::min(units, D.grid_for(reinterpret_cast<const void*>(kern), PREVIEW_BLOCK));
+    const uint32_t gstride = grid * PREVIEW_BLOCK;
+    R.gstack.ensure((size_t)(STACK_MAX - 8) * gstride);
+    D.launch("preview",
+             [&] { kern<<<grid, PREVIEW_BLOCK, 0, D.stream>>>(R.jobs.p, tr.aa_n, R.gstack.p, gstride, D.counters.p); });
     D.end_stats();
+    if (D.last_counters[CTR_OVERFLOW])
+        throw Error(FH_ERR_STATE, "traversal stack overflow");
     }
 
 // ====================================================================== serving
