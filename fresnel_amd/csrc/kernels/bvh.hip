@@ -375,9 +375,29 @@ __global__ void k_karras(const uint32_t* __restrict__ keys, const uint32_t* __re
     nodes[i].link = make_uint4(c0, c1, g0, g1);
     }
 
+// Data of the leaf at position p (primitive bounds a, b) for the 4-wide
+// search (SceneDev::leaf): neighbours in space lie next to each other.
+__device__ __forceinline__ void store_leaf(uint32_t p, float4 a, float4 b, const GeomDev* __restrict__ sphere_geoms,
+                                           float4* __restrict__ leaf, uint2* __restrict__ leaf_ref)
+    {
+    if (sphere_geoms)
+        {
+        const uint32_t slot = __float_as_uint(a.w), prim = __float_as_uint(b.w);
+        leaf[p] = sphere_geoms[slot].a[prim];
+        leaf_ref[p] = make_uint2(slot, prim);
+        }
+    else
+        {
+        leaf[2 * (size_t)p] = a;
+        leaf[2 * (size_t)p + 1] = b;
+        }
+    }
+
 // One-primitive scene: root with the leaf and an EMPTY child whose NaN box
 // fails every slab test.
-__global__ void k_single_leaf(const float4* __restrict__ lo, const float4* __restrict__ hi, Node* nodes)
+__global__ void k_single_leaf(const float4* __restrict__ lo, const float4* __restrict__ hi, Node* nodes,
+                              const GeomDev* __restrict__ sphere_geoms, float4* __restrict__ leaf,
+                              uint2* __restrict__ leaf_ref)
     {
     const float4 a = lo[0], b = hi[0];
     const float nan = __builtin_nanf("");
@@ -385,6 +405,7 @@ __global__ void k_single_leaf(const float4* __restrict__ lo, const float4* __res
     nodes[0].a_hi = make_float4(b.y, b.z, nan, nan);
     nodes[0].b_box = make_float4(nan, nan, nan, nan);
     nodes[0].link = make_uint4(LEAF | __float_as_uint(b.w), EMPTY, __float_as_uint(a.w), 0u);
+    store_leaf(0, a, b, sphere_geoms, leaf, leaf_ref);
     }
 
 // ---------------------------------------------------------------- refit
@@ -405,13 +426,15 @@ __device__ __forceinline__ void load_box(Node* n, uint32_t side, float b[6])
 
 __global__ void k_refit(const uint32_t* __restrict__ vals, const float4* __restrict__ lo,
                         const float4* __restrict__ hi, int N, Node* nodes, const uint32_t* __restrict__ parent,
-                        uint32_t* flags, float* root_box)
+                        uint32_t* flags, float* root_box, const GeomDev* __restrict__ sphere_geoms,
+                        float4* __restrict__ leaf, uint2* __restrict__ leaf_ref)
     {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= N)
         return;
     const uint32_t orig = vals[p];
     const float4 a = lo[orig], b = hi[orig];
+    store_leaf((uint32_t)p, a, b, sphere_geoms, leaf, leaf_ref);
     float box[6] = {a.x, a.y, a.z, b.x, b.y, b.z};
     uint32_t par = parent[(N - 1) + p];
     for (;;)
@@ -494,90 +517,106 @@ __device__ __forceinline__ void child_box(const Node& n, uint32_t side, float b[
     }
 
 // 4-wide node idx4[i] from inner node i of n, for the nodes at even depth:
-// idx4 is the exclusive scan of k_depth_even's flags (n + 1 entries).  With
-// sphere_geoms (a spheres-only scene) every child is stored as a centre and
-// three half extents, so the search forms each child's box as c -+ h with
-// the same operations: a leaf child holds its sphere (h = radius on every
-// axis, so c -+ h is exactly the builder's bounds), an inner child a box
-// that contains its exact box after rounding.
+// idx4 is the exclusive scan of k_depth_even's flags (n + 1 entries).  A leaf
+// child is referred to by its position in leaf order (k_karras's key order).
+// On each axis the children's boxes are rounded outwards to 8-bit steps of
+// the node's own interval, after a pad of 2^-20 of the node's largest
+// coordinate: what the search's slab test loses to rounding (search_visit).
+// An infinite or NaN end becomes one beyond every finite scene; a primitive's
+// own bounds are tested exactly at its leaf.
 __global__ void k_bvh4_fill(const Node* __restrict__ nodes, uint32_t n, const uint32_t* __restrict__ idx4,
-                            Node4* __restrict__ out, const GeomDev* __restrict__ sphere_geoms)
+                            const uint32_t* __restrict__ parent, Node4* __restrict__ out)
     {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n || idx4[i + 1] == idx4[i])
         return;
     float box[4][6];
-    uint32_t ref[4], slot[4];
+    uint32_t ref[4];
     uint32_t m = 0;
+    // leaf position of child `side` of binary node j (split position g: the
+    // children's key ranges end at g and begin at g + 1, and an inner child's
+    // index is that end); a node of two leaves is one of their positions
+    auto leaf_position = [&](uint32_t j, const uint4& l, uint32_t side)
+    {
+        uint32_t g;
+        if (l.y == EMPTY)
+            g = 0; // one-primitive scene
+        else if (!(l.x & LEAF))
+            g = l.x;
+        else if (!(l.y & LEAF))
+            g = l.y - 1;
+        else
+            g = (parent[n + j] == (j << 1)) ? j : j - 1;
+        return g + side;
+    };
     const Node a = nodes[i];
-    const uint32_t la[2] = {a.link.x, a.link.y}, ga[2] = {a.link.z, a.link.w};
+    const uint32_t la[2] = {a.link.x, a.link.y};
     for (uint32_t s = 0; s < 2; s++)
         {
-        if (la[s] & LEAF) // a leaf or EMPTY (its NaN box rejects every ray)
+        if (la[s] & LEAF) // a leaf or EMPTY (not a child)
             {
             child_box(a, s, box[m]);
-            ref[m] = la[s];
-            slot[m] = ga[s];
-            m++;
+            ref[m] = LEAF | leaf_position(i, a.link, s);
+            if (la[s] != EMPTY)
+                m++;
             continue;
             }
         const Node b = nodes[la[s]];
-        const uint32_t lb[2] = {b.link.x, b.link.y}, gb[2] = {b.link.z, b.link.w};
+        const uint32_t lb[2] = {b.link.x, b.link.y};
         for (uint32_t t = 0; t < 2; t++)
             {
             child_box(b, t, box[m]);
-            ref[m] = (lb[t] & LEAF) ? lb[t] : idx4[lb[t]];
-            slot[m] = gb[t];
+            ref[m] = (lb[t] & LEAF) ? (LEAF | leaf_position(la[s], b.link, t)) : idx4[lb[t]];
             m++;
             }
         }
-    if (sphere_geoms)
+    if (m == 1)
+        {
+        // one-primitive scene: its leaf twice
+        for (int x = 0; x < 6; x++)
+            box[1][x] = box[0][x];
+        ref[1] = ref[0];
+        m = 2;
+        }
+    constexpr float FAR = 1e18f;
+    float big = 0.0f;
+    for (uint32_t k = 0; k < m; k++)
+        for (int x = 0; x < 6; x++)
+            {
+            if (!(fabsf(box[k][x]) <= FAR))
+                box[k][x] = (x < 3) ? -FAR : FAR;
+            big = fmaxf(big, fabsf(box[k][x]));
+            }
+    const double pad = (double)NODE_PAD * big;
+    Node4 r;
+    for (int x = 0; x < 3; x++)
+        {
+        // swapped ends (a negative radius) count as the interval between them
+        double lo = 1e300, hi = -1e300;
         for (uint32_t k = 0; k < m; k++)
             {
-            if (ref[k] == EMPTY)
-                continue; // NaN box, NaN centre and extents
-            if (ref[k] & LEAF)
-                {
-                // the sphere itself: centre and radius on every axis
-                const float4 sp = sphere_geoms[slot[k]].a[ref[k] & ~LEAF];
-                box[k][0] = sp.x;
-                box[k][1] = sp.y;
-                box[k][2] = sp.z;
-                box[k][3] = sp.w;
-                box[k][4] = sp.w;
-                box[k][5] = sp.w;
-                continue;
-                }
-            // an inner box as centre c and half extents h with c - h <= lo
-            // and c + h >= hi after float rounding: h is one ulp above the
-            // rounded larger distance to c, hence above the exact distance
-            for (int x = 0; x < 3; x++)
-                {
-                const float lo = box[k][x], hi = box[k][3 + x];
-                const float c = 0.5f * lo + 0.5f * hi;
-                const float h = fmaxf(c - lo, hi - c);
-                box[k][x] = c;
-                box[k][3 + x] = __uint_as_float(__float_as_uint(h) + 1u); // h >= 0: next float up
-                }
+            lo = fmin(lo, (double)fminf(box[k][x], box[k][3 + x]));
+            hi = fmax(hi, (double)fmaxf(box[k][x], box[k][3 + x]));
             }
-    const float nan = __builtin_nanf("");
-    for (; m < 4; m++)
-        {
-        for (int k = 0; k < 6; k++)
-            box[m][k] = nan;
-        ref[m] = EMPTY;
-        slot[m] = 0;
+        // one step of head room on each side: origin and step are rounded to float
+        const float step = (float)((hi - lo + 2.0 * pad) * (1.0 / 253.0)) + 0x1p-126f;
+        const float org = (float)(lo - pad - (double)step);
+        uint32_t ql = 0, qh = 0;
+        for (uint32_t k = 0; k < m; k++)
+            {
+            const double a = (double)fminf(box[k][x], box[k][3 + x]) - pad - (double)org;
+            const double b = (double)fmaxf(box[k][x], box[k][3 + x]) + pad - (double)org;
+            const double fa = floor(a / (double)step), fb = ceil(b / (double)step);
+            ql |= (uint32_t)fmin(fmax(fa, 0.0), 255.0) << (8 * k);
+            qh |= (uint32_t)fmin(fmax(fb, 0.0), 255.0) << (8 * k);
+            }
+        r.o[x] = org;
+        r.s[x] = step;
+        r.qlo[x] = ql;
+        r.qhi[x] = qh;
         }
-    Node4 r;
-    for (int q = 0; q < 2; q++)
-        {
-        const float* b0 = box[2 * q];
-        const float* b1 = box[2 * q + 1];
-        r.pair[q].a_lo = make_float4(b0[0], b0[1], b0[2], b0[3]);
-        r.pair[q].a_hi = make_float4(b0[4], b0[5], b1[0], b1[1]);
-        r.pair[q].b_box = make_float4(b1[2], b1[3], b1[4], b1[5]);
-        r.pair[q].link = make_uint4(ref[2 * q], ref[2 * q + 1], slot[2 * q], slot[2 * q + 1]);
-        }
+    for (uint32_t k = 0; k < 4; k++)
+        r.ref[k] = (k < m) ? ref[k] : EMPTY;
     out[idx4[i]] = r;
     }
 

@@ -54,6 +54,31 @@ __device__ __forceinline__ bool better(float t, uint32_t g, uint32_t p, const Hi
     return lt | (eq & (g_lt | (g_eq & p_lt)));
     }
 
+// Element i of an array in global memory (a direct global load, not a flat one).
+typedef float F4v __attribute__((ext_vector_type(4)));
+typedef uint32_t U4v __attribute__((ext_vector_type(4)));
+typedef uint32_t U2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float4 ldg(const float4* p, size_t i)
+    {
+    const F4v v = ((const F4v __attribute__((address_space(1)))*)p)[i];
+    return make_float4(v.x, v.y, v.z, v.w);
+    }
+__device__ __forceinline__ uint4 ldg(const uint4* p, size_t i)
+    {
+    const U4v v = ((const U4v __attribute__((address_space(1)))*)p)[i];
+    return make_uint4(v.x, v.y, v.z, v.w);
+    }
+__device__ __forceinline__ uint2 ldg(const uint2* p, size_t i)
+    {
+    const U2v v = ((const U2v __attribute__((address_space(1)))*)p)[i];
+    return make_uint2(v.x, v.y);
+    }
+__device__ __forceinline__ void stg(uint2* p, size_t i, uint2 e)
+    {
+    U2v v = {e.x, e.y};
+    ((U2v __attribute__((address_space(1)))*)p)[i] = v;
+    }
+
 // Stack with the top SS entries in LDS (interleaved by thread) and the rest
 // in a per-thread global region.
 template<int SS> struct LdsStack
@@ -68,7 +93,7 @@ template<int SS> struct LdsStack
         if (sp < SS)
             lds[sp * lstride] = e;
         else if (sp < STACK_MAX)
-            glob[(sp - SS) * gstride] = e;
+            stg(glob, (size_t)(sp - SS) * gstride, e);
         else
             {
             err = 1;
@@ -76,10 +101,39 @@ template<int SS> struct LdsStack
             }
         sp++;
         }
+    // Push the entries whose key is finite, the first argument pair first
+    // (sorted by descending key, so the finite ones are the last).  With room
+    // in LDS for all three there is no branch: each is written where the next
+    // entry goes, and stays when its key is finite.
+    __device__ __forceinline__ void push3(uint32_t n3, float k3, uint32_t n2, float k2, uint32_t n1, float k1,
+                                          uint32_t& err)
+        {
+        const float inf = __builtin_huge_valf();
+        if (sp + 3 <= SS)
+            {
+            lds[sp * lstride] = make_uint2(n3, __float_as_uint(k3));
+            sp += (k3 < inf) ? 1u : 0u;
+            lds[sp * lstride] = make_uint2(n2, __float_as_uint(k2));
+            sp += (k2 < inf) ? 1u : 0u;
+            lds[sp * lstride] = make_uint2(n1, __float_as_uint(k1));
+            sp += (k1 < inf) ? 1u : 0u;
+            return;
+            }
+        if (k3 < inf)
+            push(n3, k3, err);
+        if (k2 < inf)
+            push(n2, k2, err);
+        if (k1 < inf)
+            push(n1, k1, err);
+        }
     __device__ __forceinline__ void pop(uint32_t& n, float& t)
         {
         sp--;
-        const uint2 e = (sp < SS) ? lds[sp * lstride] : glob[(sp - SS) * gstride];
+        uint2 e;
+        if (sp < SS)
+            e = lds[sp * lstride];
+        else
+            e = ldg(glob, (size_t)(sp - SS) * gstride);
         n = e.x;
         t = __uint_as_float(e.y);
         }
@@ -96,6 +150,17 @@ struct LocalStack
             s[sp++] = make_uint2(n, __float_as_uint(t));
         else
             err = 1;
+        }
+    __device__ __forceinline__ void push3(uint32_t n3, float k3, uint32_t n2, float k2, uint32_t n1, float k1,
+                                          uint32_t& err)
+        {
+        const float inf = __builtin_huge_valf();
+        if (k3 < inf)
+            push(n3, k3, err);
+        if (k2 < inf)
+            push(n2, k2, err);
+        if (k1 < inf)
+            push(n1, k1, err);
         }
     __device__ __forceinline__ void pop(uint32_t& n, float& t)
         {
@@ -125,7 +190,7 @@ __device__ __forceinline__ bool leaf_test(const GeomDev& g, uint32_t prim, v3 o,
 
 typedef const Node __attribute__((address_space(1))) GlobalNode;
 
-// Closest-hit traversal state of one ray.
+// State of a ray's search of the binary hierarchy (below a tile-list subtree).
 struct TraceState
     {
     v3 o, d, inv;
@@ -133,184 +198,10 @@ struct TraceState
     float margin;
     HitT best;
     uint32_t node;
-    bool sph; // 4-wide leaf children hold spheres
     };
 
-template<class Stack>
-__device__ __forceinline__ void trace_begin(const SceneDev& sc, v3 o, v3 d, float tnear, TraceState& r, Stack& st)
-    {
-    r.o = o;
-    r.d = d;
-    r.inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    r.tnear = tnear;
-    r.margin = sc.cull_margin;
-    r.best.t = __builtin_huge_valf();
-    r.best.geom = EMPTY;
-    r.best.prim = EMPTY;
-    r.node = sc.root;
-    r.sph = sc.sphere_leaves != 0;
-    st.sp = 0;
-    }
-
-// Primitive test of a leaf child that passed the slab and cull tests.
-template<bool COUNT, uint32_t TYPES>
-__device__ __forceinline__ void visit_leaf(const GeomDev* __restrict__ geoms, uint32_t ref, uint32_t slot,
-                                           TraceState& r, uint32_t& n_prims)
-    {
-    const uint32_t prim = ref & ~LEAF;
-    float t;
-    if (COUNT)
-        n_prims++;
-    if (leaf_test<TYPES>(geoms[slot], prim, r.o, r.d, r.tnear, t) && better(t, slot, prim, r.best))
-        {
-        r.best.t = t;
-        r.best.geom = slot;
-        r.best.prim = prim;
-        }
-    }
-
-// Sort two (key, node, bound) entries by key.
-__device__ __forceinline__ void order2(float& ka, uint32_t& na, float& ca, float& kb, uint32_t& nb, float& cb)
-    {
-    const bool sw = kb < ka;
-    const float k = sw ? kb : ka, c = sw ? cb : ca;
-    const uint32_t n = sw ? nb : na;
-    kb = sw ? ka : kb;
-    nb = sw ? na : nb;
-    cb = sw ? ca : cb;
-    ka = k;
-    na = n;
-    ca = c;
-    }
-
-// One node visit of the closest-hit search over the 4-wide hierarchy: the
-// primitives of leaf children are tested, the nearest hit inner child is
-// visited next and the others are pushed, farthest first.  Returns false when
-// the search is complete.  The closest hit is the smallest (t, geometry,
-// primitive) over the primitives whose bounds pass the slab test with
-// tmax >= tnear; a subtree is culled when the lower bound of its primitives'
-// distances (cull_bound) exceeds the closest hit, so neither the hierarchy
-// nor the visiting order changes the result.
-template<class Stack, bool COUNT, uint32_t TYPES>
-__device__ __forceinline__ bool trace_visit4(const Node4* __restrict__ nodes, const GeomDev* __restrict__ geoms,
-                                            TraceState& r, Stack& st, uint32_t& n_nodes, uint32_t& n_prims,
-                                            uint32_t& err)
-    {
-    if (r.node == EMPTY)
-        return false;
-    if (COUNT)
-        n_nodes++;
-    // spheres-only kernels always see sphere leaves (checked on the host)
-    const bool sph = (TYPES == T_SPHERES) || r.sph;
-    float tmin[4], cb[4];
-    bool h[4];
-    uint32_t ch[4];
-#pragma unroll
-    for (int q = 0; q < 2; q++)
-        {
-        // one child pair: global address space, direct global loads
-        const GlobalNode* np = (const GlobalNode*)(&nodes[r.node].pair[q]);
-        const float4 A = make_float4(np->a_lo.x, np->a_lo.y, np->a_lo.z, np->a_lo.w);
-        const float4 B = make_float4(np->a_hi.x, np->a_hi.y, np->a_hi.z, np->a_hi.w);
-        const float4 C = make_float4(np->b_box.x, np->b_box.y, np->b_box.z, np->b_box.w);
-        const uint4 lk = make_uint4(np->link.x, np->link.y, np->link.z, np->link.w);
-        const float bx[2][6] = {{A.x, A.y, A.z, A.w, B.x, B.y}, {B.z, B.w, C.x, C.y, C.z, C.w}};
-        const uint32_t ref[2] = {lk.x, lk.y}, slot[2] = {lk.z, lk.w};
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-            {
-            const int k = 2 * q + c;
-            // with sphere leaves every child is a centre and half extents
-            // (k_bvh4_fill): a sphere leaf's box is centre -+ radius, as the
-            // builder bounds it (GeometrySphere.cc:60-73)
-            float x0 = bx[c][0], y0 = bx[c][1], z0 = bx[c][2], x1 = bx[c][3], y1 = bx[c][4], z1 = bx[c][5];
-            if (sph)
-                {
-                x0 = bx[c][0] - bx[c][3];
-                x1 = bx[c][0] + bx[c][3];
-                y0 = bx[c][1] - bx[c][4];
-                y1 = bx[c][1] + bx[c][4];
-                z0 = bx[c][2] - bx[c][5];
-                z1 = bx[c][2] + bx[c][5];
-                }
-            float tmax;
-            slab(r.o, r.inv, x0, y0, z0, x1, y1, z1, tmin[k], tmax);
-            cb[k] = cull_bound(tmin[k], tmax, r.margin);
-            h[k] = (tmin[k] <= tmax) && (tmax >= r.tnear) && !(cb[k] > r.best.t);
-            ch[k] = ref[c];
-            }
-        // leaf children of this pair
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-            {
-            const int k = 2 * q + c;
-            if (h[k] && (ref[c] & LEAF))
-                {
-                if (sph)
-                    {
-                    // the sphere is in the node: no memory access
-                    const uint32_t prim = ref[c] & ~LEAF;
-                    float t, de;
-                    bool first;
-                    if (COUNT)
-                        n_prims++;
-                    if (sphere_t(r.o, r.d, mk3(bx[c][0], bx[c][1], bx[c][2]), bx[c][3], t, de, first)
-                        && (r.tnear < t) && better(t, slot[c], prim, r.best))
-                        {
-                        r.best.t = t;
-                        r.best.geom = slot[c];
-                        r.best.prim = prim;
-                        }
-                    }
-                else
-                    visit_leaf<COUNT, TYPES>(geoms, ref[c], slot[c], r, n_prims);
-                h[k] = false;
-                }
-            }
-        }
-    // inner children still open, nearest entry first
-    float key[4];
-    uint32_t nd[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-        {
-        const bool open = h[k] && !(cb[k] > r.best.t);
-        key[k] = open ? tmin[k] : __builtin_huge_valf();
-        nd[k] = open ? ch[k] : EMPTY;
-        }
-    order2(key[0], nd[0], cb[0], key[1], nd[1], cb[1]);
-    order2(key[2], nd[2], cb[2], key[3], nd[3], cb[3]);
-    order2(key[0], nd[0], cb[0], key[2], nd[2], cb[2]);
-    order2(key[1], nd[1], cb[1], key[3], nd[3], cb[3]);
-    order2(key[1], nd[1], cb[1], key[2], nd[2], cb[2]);
-    if (nd[0] != EMPTY)
-        {
-#pragma unroll
-        for (int k = 3; k >= 1; k--)
-            if (nd[k] != EMPTY)
-                st.push(nd[k], cb[k], err);
-        r.node = nd[0];
-        return true;
-        }
-    while (st.sp > 0)
-        {
-        uint32_t n;
-        float tm;
-        st.pop(n, tm);
-        if (!(tm > r.best.t))
-            {
-            r.node = n;
-            return true;
-            }
-        }
-    r.node = EMPTY;
-    return false;
-    }
-
 // One node visit of the closest-hit search over the binary hierarchy (the
-// kernels for scenes with other primitive types, whose larger intersectors
-// leave no registers for 4-wide nodes): the primitives of leaf children
-// are tested, the nearer hit inner child is visited next and the farther one
+// subtrees of tile lists): the primitives of leaf children are tested, the nearer hit inner child is visited next and the farther one
 // pushed.  Returns false when the search is complete.  The closest hit is
 // the smallest (t, geometry, primitive) over the primitives whose bounds pass
 // the slab test with tmax >= tnear; a subtree is culled when the lower bound
@@ -399,114 +290,13 @@ __device__ __forceinline__ bool trace_visit2(const Node* __restrict__ nodes, con
     return false;
     }
 
-// One node visit of the closest-hit search: spheres-only kernels search the
-// 4-wide hierarchy, the others the binary one (same result either way).
-template<class Stack, bool COUNT, uint32_t TYPES>
-__device__ __forceinline__ bool trace_visit(const SceneDev& sc, TraceState& r, Stack& st, uint32_t& n_nodes,
-                                            uint32_t& n_prims, uint32_t& err)
-    {
-    if constexpr (TYPES == T_SPHERES)
-        return trace_visit4<Stack, COUNT, TYPES>(sc.nodes4, sc.geoms, r, st, n_nodes, n_prims, err);
-    else
-        return trace_visit2<Stack, COUNT, TYPES>(sc.nodes, sc.geoms, r, st, n_nodes, n_prims, err);
-    }
-
-template<class Stack, bool COUNT, uint32_t TYPES = T_ALL>
-__device__ inline void trace_closest(const SceneDev& sc, v3 o, v3 d, float tnear, HitT& best, Stack& st,
-                                     uint32_t& n_nodes, uint32_t& n_prims, uint32_t& err)
-    {
-    TraceState r;
-    trace_begin(sc, o, d, tnear, r, st);
-    while (trace_visit<Stack, COUNT, TYPES>(sc, r, st, n_nodes, n_prims, err))
-        {
-        }
-    best = r.best;
-    }
-
-// One node visit of the binary-hierarchy search with the primitive tests
-// postponed: leaf children that pass the slab and cull tests are appended to
-// the lane's pending list (ps, pp; np entries, at most two per visit) instead
-// of being tested; inner children are visited or pushed as in trace_visit2.
-template<class Stack, bool COUNT>
-__device__ __forceinline__ void visit2_collect(const Node* __restrict__ nodes, TraceState& r, Stack& st,
-                                               uint32_t (&ps)[2], uint32_t (&pp)[2], uint32_t& np,
-                                               uint32_t& n_nodes, uint32_t& err)
-    {
-    const GlobalNode* n = (const GlobalNode*)(nodes + r.node);
-    const float4 A = make_float4(n->a_lo.x, n->a_lo.y, n->a_lo.z, n->a_lo.w);
-    const float4 B = make_float4(n->a_hi.x, n->a_hi.y, n->a_hi.z, n->a_hi.w);
-    const float4 C = make_float4(n->b_box.x, n->b_box.y, n->b_box.z, n->b_box.w);
-    const uint4 lk = make_uint4(n->link.x, n->link.y, n->link.z, n->link.w);
-    if (COUNT)
-        n_nodes++;
-    float t0min, t0max, t1min, t1max;
-    slab(r.o, r.inv, A.x, A.y, A.z, A.w, B.x, B.y, t0min, t0max);
-    slab(r.o, r.inv, B.z, B.w, C.x, C.y, C.z, C.w, t1min, t1max);
-    const float c0 = cull_bound(t0min, t0max, r.margin);
-    const float c1 = cull_bound(t1min, t1max, r.margin);
-    bool h0 = (t0min <= t0max) && (t0max >= r.tnear) && !(c0 > r.best.t);
-    bool h1 = (t1min <= t1max) && (t1max >= r.tnear) && !(c1 > r.best.t);
-    if (h0 && (lk.x & LEAF))
-        {
-        ps[0] = lk.z;
-        pp[0] = lk.x & ~LEAF;
-        np = 1;
-        h0 = false;
-        }
-    if (h1 && (lk.y & LEAF))
-        {
-        // constant indices keep the list in registers
-        if (np == 0)
-            {
-            ps[0] = lk.w;
-            pp[0] = lk.y & ~LEAF;
-            }
-        else
-            {
-            ps[1] = lk.w;
-            pp[1] = lk.y & ~LEAF;
-            }
-        np++;
-        h1 = false;
-        }
-    if (h0 && h1)
-        {
-        const bool swap = t1min < t0min;
-        st.push(swap ? lk.x : lk.y, swap ? c0 : c1, err);
-        r.node = swap ? lk.y : lk.x;
-        return;
-        }
-    if (h0 || h1)
-        {
-        r.node = h0 ? lk.x : lk.y;
-        return;
-        }
-    r.node = EMPTY;
-    while (st.sp > 0)
-        {
-        uint32_t nn;
-        float tm;
-        st.pop(nn, tm);
-        if (!(tm > r.best.t))
-            {
-            r.node = nn;
-            return;
-            }
-        }
-    }
-
-// Postponed primitive tests of type G: the lanes whose pending entry k is a
-// primitive of that type run its intersector together.
+// Intersector of one primitive of type G, if the state's types hold it.
 template<uint32_t G, uint32_t TYPES, bool COUNT>
-__device__ __forceinline__ void test_pending(const GeomDev* __restrict__ geoms, TraceState& r, bool has, uint32_t ty,
-                                             uint32_t slot, uint32_t prim, uint32_t& n_prims)
+__device__ __forceinline__ void test_binary(const GeomDev* __restrict__ geoms, TraceState& r, uint32_t ty,
+                                            uint32_t slot, uint32_t prim, uint32_t& n_prims)
     {
     if constexpr ((TYPES & (1u << G)) != 0)
-        {
-        const bool mine = has && ty == G;
-        if (__ballot(mine) == 0)
-            return;
-        if (mine)
+        if (ty == G)
             {
             float t;
             if (COUNT)
@@ -519,56 +309,423 @@ __device__ __forceinline__ void test_pending(const GeomDev* __restrict__ geoms, 
                 r.best.prim = prim;
                 }
             }
-        }
     }
 
-// Closest hit over the binary hierarchy for scenes of several primitive
-// types, one ray per lane.  A lane that reaches leaves keeps them pending and
-// waits; once the waiting lanes are at least twice as many as those still
-// searching (or none can go on), the pending primitives are tested one
-// geometry type at a time,
-// so each intersector runs once for all the lanes that need it instead of a
-// few lanes at a time per node visit.  Culling meanwhile uses the closest hit
-// found so far, which only prunes less; every primitive whose bounds pass the
-// slab test and that could still win is tested, so the result is the same
-// (t, geometry, primitive) minimum as trace_closest's.
+// Closest hit of each lane's ray by the binary search from the root: for each
+// lane the visits, tests and comparisons of trace_visit2 in the same order,
+// but a lane that reaches leaves stops in the middle of its visit until the
+// waiting lanes are twice those that can go on, and the primitive tests run
+// for all of them, one type at a time (20,000 polyhedra, 1280 x 720, 64
+// samples: 18.6 ms with the tests on the spot, 16.8 so).
 template<class Stack, bool COUNT, uint32_t TYPES>
-__device__ inline void trace_closest_grouped(const SceneDev& sc, v3 o, v3 d, float tnear, HitT& best, Stack& st,
-                                             uint32_t& n_nodes, uint32_t& n_prims, uint32_t& err)
+__device__ inline void trace_binary(const SceneDev& sc, v3 o, v3 d, float tnear, HitT& best, Stack& st,
+                                    uint32_t& n_nodes, uint32_t& n_prims, uint32_t& err)
     {
+    const Node* __restrict__ nodes = sc.nodes;
+    const GeomDev* __restrict__ geoms = sc.geoms;
     TraceState r;
-    trace_begin(sc, o, d, tnear, r, st);
-    uint32_t ps[2] = {0, 0}, pp[2] = {0, 0};
-    uint32_t np = 0;
+    r.o = o;
+    r.d = d;
+    r.inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    r.tnear = tnear;
+    r.margin = sc.cull_margin;
+    r.best.t = __builtin_huge_valf();
+    r.best.geom = EMPTY;
+    r.best.prim = EMPTY;
+    r.node = sc.root;
+    st.sp = 0;
+    bool wait = false, h0 = false, h1 = false, swap = false;
+    float c0 = 0.0f, c1 = 0.0f;
+    uint4 lk = make_uint4(0, 0, 0, 0);
+    // the rest of a visit once its leaves are tested
+    auto advance = [&]()
+    {
+        const bool a = h0 && !(lk.x & LEAF) && !(c0 > r.best.t);
+        const bool b = h1 && !(lk.y & LEAF) && !(c1 > r.best.t);
+        if (a && b)
+            st.push(swap ? lk.x : lk.y, swap ? c0 : c1, err);
+        if (a || b)
+            {
+            r.node = (b && (!a || swap)) ? lk.y : lk.x;
+            return;
+            }
+        r.node = EMPTY;
+        while (st.sp > 0)
+            {
+            uint32_t n;
+            float tm;
+            st.pop(n, tm);
+            if (!(tm > r.best.t))
+                {
+                r.node = n;
+                return;
+                }
+            }
+    };
     for (;;)
         {
         for (;;)
             {
-            const bool go = r.node != EMPTY && np == 0;
+            const bool go = r.node != EMPTY && !wait;
             const uint32_t n_go = (uint32_t)__popcll(__ballot(go));
-            const uint32_t n_wait = (uint32_t)__popcll(__ballot(np != 0));
+            const uint32_t n_wait = (uint32_t)__popcll(__ballot(wait));
             if (n_go == 0 || n_wait >= 2 * n_go)
                 break;
             if (go)
-                visit2_collect<Stack, COUNT>(sc.nodes, r, st, ps, pp, np, n_nodes, err);
+                {
+                const float4* np = (const float4*)(nodes + r.node);
+                const float4 A = ldg(np, 0), B = ldg(np, 1), C = ldg(np, 2);
+                lk = ldg((const uint4*)np, 3);
+                if (COUNT)
+                    n_nodes++;
+                float t0min, t0max, t1min, t1max;
+                slab(r.o, r.inv, A.x, A.y, A.z, A.w, B.x, B.y, t0min, t0max);
+                slab(r.o, r.inv, B.z, B.w, C.x, C.y, C.z, C.w, t1min, t1max);
+                c0 = cull_bound(t0min, t0max, r.margin);
+                c1 = cull_bound(t1min, t1max, r.margin);
+                h0 = (t0min <= t0max) && (t0max >= r.tnear) && !(c0 > r.best.t);
+                h1 = (t1min <= t1max) && (t1max >= r.tnear) && !(c1 > r.best.t);
+                swap = t1min < t0min;
+                wait = (h0 && (lk.x & LEAF)) || (h1 && (lk.y & LEAF));
+                if (!wait)
+                    advance();
+                }
             }
-        if (__ballot(np != 0) == 0)
+        if (__ballot(wait) == 0)
             break;
-#pragma unroll
         for (uint32_t k = 0; k < 2; k++)
             {
-            const bool has = np > k;
-            const uint32_t slot = ps[k], prim = pp[k];
-            const uint32_t ty = has ? sc.geoms[slot].type : 0xffu;
-            test_pending<G_SPHERE, TYPES, COUNT>(sc.geoms, r, has, ty, slot, prim, n_prims);
-            test_pending<G_CYLINDER, TYPES, COUNT>(sc.geoms, r, has, ty, slot, prim, n_prims);
-            test_pending<G_POLYHEDRON, TYPES, COUNT>(sc.geoms, r, has, ty, slot, prim, n_prims);
-            test_pending<G_MESH, TYPES, COUNT>(sc.geoms, r, has, ty, slot, prim, n_prims);
-            test_pending<G_POLYGON, TYPES, COUNT>(sc.geoms, r, has, ty, slot, prim, n_prims);
+            const uint32_t ref = k ? lk.y : lk.x, slot = k ? lk.w : lk.z;
+            const uint32_t ty = (wait && (k ? h1 : h0) && (ref & LEAF)) ? geoms[slot].type : 0xffu;
+            const uint32_t prim = ref & ~LEAF;
+            test_binary<G_SPHERE, TYPES, COUNT>(geoms, r, ty, slot, prim, n_prims);
+            test_binary<G_CYLINDER, TYPES, COUNT>(geoms, r, ty, slot, prim, n_prims);
+            test_binary<G_POLYHEDRON, TYPES, COUNT>(geoms, r, ty, slot, prim, n_prims);
+            test_binary<G_MESH, TYPES, COUNT>(geoms, r, ty, slot, prim, n_prims);
+            test_binary<G_POLYGON, TYPES, COUNT>(geoms, r, ty, slot, prim, n_prims);
             }
-        np = 0;
+        if (wait)
+            {
+            advance();
+            wait = false;
+            }
         }
     best = r.best;
+    }
+
+// ---------------------------------------------------------------- 4-wide search
+// Closest-hit search over the 4-wide hierarchy.  A ray walks the nodes with a
+// cheap test that only has to be conservative, and the primitives it reaches
+// are tested later, many lanes together:
+//   * a child box is 8-bit steps of the node's interval (k_bvh4_fill); the
+//     ray's direction signs pick the near and far ends, so an axis of a
+//     child's slab interval is two byte conversions and two fmas.  The node's
+//     pad and the ray's (2^-20 of the largest coordinate of node and origin
+//     each, against rounding errors of at most 7 and 6 x 2^-24 of them) make
+//     the interval contain, on every axis, the float slab interval
+//     (lo - o) * inv of every primitive inside;
+//   * the exact slab gate of a primitive's own bounds and its intersector run
+//     at the leaf step.  Leaf children are sorted and pushed like inner ones;
+//     a lane that takes one waits until enough lanes hold one.
+// A child is culled when its key, max(tmin, 0) - CULL_K tmax, exceeds the
+// closest hit plus the scene's margin (cull_bound with the margin moved to
+// the other side; CULL_K's factor of two covers the roundings of key and sum).
+// So every primitive whose bounds pass the slab test and that could still win
+// is tested, and the result is the smallest (t, geometry, primitive) whatever
+// the hierarchy and the order.
+//
+// Bound by VALU issue (99 % on the lattice) with under half the lanes active.
+// Exact boxes and leaf tests on the spot took about 450 instructions per
+// visit, with a few lanes in the sphere solves; this form takes about 160 per
+// visit and 100 per leaf step.  With 128-byte nodes of float centres and half
+// extents (seven 16-byte loads per visit instead of four) the loads bound it:
+// 11.6 ms on the lattice against 9.2.
+//
+// What the search reads of a scene.  UNI (one scene for the whole wavefront):
+// the pointers are read once, through scalar loads, and stay in scalar
+// registers; otherwise each lane reads its own scene's record when it needs
+// it, which costs every node visit a load that its node's loads wait for.
+template<bool UNI> struct SearchScene;
+template<> struct SearchScene<true>
+    {
+    const Node4* n4;
+    const float4* lf;
+    const uint2* lr;
+    const GeomDev* g;
+    __device__ __forceinline__ SearchScene(const SceneDev& s) : n4(s.nodes4), lf(s.leaf), lr(s.leaf_ref), g(s.geoms) { }
+    __device__ __forceinline__ const Node4* nodes4() const { return n4; }
+    __device__ __forceinline__ const float4* leaf() const { return lf; }
+    __device__ __forceinline__ const uint2* leaf_ref() const { return lr; }
+    __device__ __forceinline__ const GeomDev* geoms() const { return g; }
+    };
+template<> struct SearchScene<false>
+    {
+    const SceneDev& s;
+    __device__ __forceinline__ SearchScene(const SceneDev& sc) : s(sc) { }
+    __device__ __forceinline__ const Node4* nodes4() const { return s.nodes4; }
+    __device__ __forceinline__ const float4* leaf() const { return s.leaf; }
+    __device__ __forceinline__ const uint2* leaf_ref() const { return s.leaf_ref; }
+    __device__ __forceinline__ const GeomDev* geoms() const { return s.geoms; }
+    };
+
+struct Search
+    {
+    v3 o, d, inv;     // the ray; exact reciprocals for the primitives' gates
+    v3 ic, near, far; // node tests: bounded reciprocals, -o * ic less and plus the pad
+    float tnear;
+    float margin;
+    float cull;       // best.t + margin
+    HitT best;        // spheres-only: prim is the leaf position until search_end
+    uint32_t cur;     // inner node, LEAF | leaf position, or EMPTY: done
+    };
+
+// Reciprocal of a direction component for the node tests.  Below 2^-60 it is
+// taken as 2^60: a box the origin lies beside by more than the pads is missed,
+// and inside one the interval reaches 2^40 times the largest coordinate, past
+// every hit.
+__device__ __forceinline__ float node_rcp(float d, float inv)
+    {
+    return (fabsf(d) < 0x1p-60f) ? copysignf(0x1p60f, d) : inv;
+    }
+
+template<class Stack>
+__device__ __forceinline__ void search_begin(const SceneDev& sc, v3 o, v3 d, float tnear, Search& r, Stack& st)
+    {
+    r.o = o;
+    r.d = d;
+    r.inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
+    r.ic = mk3(node_rcp(d.x, r.inv.x), node_rcp(d.y, r.inv.y), node_rcp(d.z, r.inv.z));
+    const v3 n = mk3(-(o.x * r.ic.x), -(o.y * r.ic.y), -(o.z * r.ic.z));
+    const float om = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) * NODE_PAD;
+    const v3 pad = mk3(om * fabsf(r.ic.x), om * fabsf(r.ic.y), om * fabsf(r.ic.z));
+    r.near = n - pad;
+    r.far = n + pad;
+    r.tnear = tnear;
+    r.margin = sc.cull_margin;
+    r.cull = __builtin_huge_valf();
+    r.best.t = __builtin_huge_valf();
+    r.best.geom = EMPTY;
+    r.best.prim = EMPTY;
+    r.cur = sc.root;
+    st.sp = 0;
+    }
+
+// Next entry of the stack that is not culled (EMPTY: the search is complete).
+template<class Stack> __device__ __forceinline__ void search_pop(Search& r, Stack& st)
+    {
+    r.cur = EMPTY;
+    while (st.sp > 0)
+        {
+        uint32_t n;
+        float key;
+        st.pop(n, key);
+        if (!(key > r.cull))
+            {
+            r.cur = n;
+            return;
+            }
+        }
+    }
+
+__device__ __forceinline__ void order2(float& ka, uint32_t& na, float& kb, uint32_t& nb)
+    {
+    const bool sw = kb < ka;
+    const float k = sw ? kb : ka;
+    const uint32_t n = sw ? nb : na;
+    kb = sw ? ka : kb;
+    nb = sw ? na : nb;
+    ka = k;
+    na = n;
+    }
+
+// One node visit: the nearest open child is taken next, the others are pushed,
+// farthest first.
+template<class Stack, bool COUNT>
+__device__ __forceinline__ void search_visit(const Node4* __restrict__ nodes, Search& r, Stack& st, uint32_t& n_nodes,
+                                             uint32_t& err)
+    {
+    if (COUNT)
+        n_nodes++;
+    const uint4* np = (const uint4*)(nodes + r.cur);
+    const uint4 A = ldg(np, 0), B = ldg(np, 1), C = ldg(np, 2), ref = ldg(np, 3);
+    // A: origin, step x | B: step y z, low x y | C: low z, high x y z
+    const float ox = __uint_as_float(A.x), oy = __uint_as_float(A.y), oz = __uint_as_float(A.z);
+    const float sx = __uint_as_float(A.w) * r.ic.x, sy = __uint_as_float(B.x) * r.ic.y,
+                sz = __uint_as_float(B.y) * r.ic.z;
+    const float nx = __builtin_fmaf(ox, r.ic.x, r.near.x), fx = __builtin_fmaf(ox, r.ic.x, r.far.x);
+    const float ny = __builtin_fmaf(oy, r.ic.y, r.near.y), fy = __builtin_fmaf(oy, r.ic.y, r.far.y);
+    const float nz = __builtin_fmaf(oz, r.ic.z, r.near.z), fz = __builtin_fmaf(oz, r.ic.z, r.far.z);
+    const bool px = r.ic.x >= 0.0f, py = r.ic.y >= 0.0f, pz = r.ic.z >= 0.0f;
+    const uint32_t qnx = px ? B.z : C.y, qfx = px ? C.y : B.z;
+    const uint32_t qny = py ? B.w : C.z, qfy = py ? C.z : B.w;
+    const uint32_t qnz = pz ? C.x : C.w, qfz = pz ? C.w : C.x;
+    uint32_t nd[4] = {ref.x, ref.y, ref.z, ref.w};
+    float key[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        {
+        auto byte = [k](uint32_t q) { return (float)((q >> (8 * k)) & 0xffu); };
+        const float tx = __builtin_fmaf(byte(qnx), sx, nx), ux = __builtin_fmaf(byte(qfx), sx, fx);
+        const float ty = __builtin_fmaf(byte(qny), sy, ny), uy = __builtin_fmaf(byte(qfy), sy, fy);
+        const float tz = __builtin_fmaf(byte(qnz), sz, nz), uz = __builtin_fmaf(byte(qfz), sz, fz);
+        const float lo = fmaxf(fmaxf(fmaxf(tx, ty), tz), 0.0f);
+        const float hi = fminf(fminf(ux, uy), uz);
+        const float q = __builtin_fmaf(-CULL_K, hi, lo);
+        const bool open = (lo <= hi) & !(q > r.cull) & (k < 2 || nd[k] != EMPTY);
+        key[k] = open ? q : __builtin_huge_valf();
+        }
+    order2(key[0], nd[0], key[1], nd[1]);
+    order2(key[2], nd[2], key[3], nd[3]);
+    order2(key[0], nd[0], key[2], nd[2]);
+    order2(key[1], nd[1], key[3], nd[3]);
+    order2(key[1], nd[1], key[2], nd[2]);
+    if (key[0] < __builtin_huge_valf())
+        {
+        st.push3(nd[3], key[3], nd[2], key[2], nd[1], key[1], err);
+        r.cur = nd[0];
+        }
+    else
+        search_pop(r, st);
+    }
+
+// Leaf step of the lanes whose cur is a leaf (in a spheres-only scene): the
+// exact slab gate of the sphere's bounds as the builder computes them
+// (GeometrySphere.cc:60-73), then the sphere test.
+template<bool COUNT, bool UNI>
+__device__ __forceinline__ void search_sphere(const SearchScene<UNI>& sc, Search& r, uint32_t& n_prims)
+    {
+    const uint32_t p = r.cur & ~LEAF;
+    const float4 s = ldg(sc.leaf(), p);
+    float tmin, tmax;
+    slab(r.o, r.inv, s.x - s.w, s.y - s.w, s.z - s.w, s.x + s.w, s.y + s.w, s.z + s.w, tmin, tmax);
+    if (!((tmin <= tmax) && (tmax >= r.tnear)))
+        return;
+    if (COUNT)
+        n_prims++;
+    float t, de;
+    bool first;
+    if (!sphere_t(r.o, r.d, mk3(s.x, s.y, s.z), s.w, t, de, first) || !(r.tnear < t))
+        return;
+    bool win = t < r.best.t;
+    if (t == r.best.t)
+        {
+        win = true;
+        if (r.best.prim != EMPTY)
+            {
+            const uint2 a = ldg(sc.leaf_ref(), p), b = ldg(sc.leaf_ref(), r.best.prim);
+            win = a.x < b.x || (a.x == b.x && a.y < b.y);
+            }
+        }
+    if (win)
+        {
+        r.best.t = t;
+        r.best.prim = p;
+        r.cull = t + r.margin;
+        }
+    }
+
+// Primitive tests of type G: the lanes that hold a primitive of that type run
+// its intersector together.
+template<uint32_t G, uint32_t TYPES, bool COUNT>
+__device__ __forceinline__ void test_type(const GeomDev* __restrict__ geoms, Search& r, uint32_t ty, uint32_t slot,
+                                          uint32_t prim, uint32_t& n_prims)
+    {
+    if constexpr ((TYPES & (1u << G)) != 0)
+        if (ty == G)
+            {
+            float t;
+            if (COUNT)
+                n_prims++;
+            if (intersect_prim<false, 1u << G>(geoms[slot], prim, r.o, r.d, r.tnear, t, nullptr)
+                && better(t, slot, prim, r.best))
+                {
+                r.best.t = t;
+                r.best.geom = slot;
+                r.best.prim = prim;
+                r.cull = t + r.margin;
+                }
+            }
+    }
+
+// Leaf step in other scenes (the leaf array's form depends on the scene:
+// kernels of other types are never given a spheres-only scene): the gate with the stored bounds, then one
+// geometry type at a time.
+template<uint32_t TYPES, bool COUNT, bool UNI>
+__device__ __forceinline__ void search_mixed(const SearchScene<UNI>& sc, Search& r, uint32_t& n_prims)
+    {
+    const uint32_t p = r.cur & ~LEAF;
+    const float4 a = ldg(sc.leaf(), 2 * (size_t)p), b = ldg(sc.leaf(), 2 * (size_t)p + 1);
+    float tmin, tmax;
+    slab(r.o, r.inv, a.x, a.y, a.z, b.x, b.y, b.z, tmin, tmax);
+    if (!((tmin <= tmax) && (tmax >= r.tnear)))
+        return;
+    const uint32_t slot = __float_as_uint(a.w), prim = __float_as_uint(b.w);
+    const uint32_t ty = sc.geoms()[slot].type;
+    test_type<G_SPHERE, TYPES, COUNT>(sc.geoms(), r, ty, slot, prim, n_prims);
+    test_type<G_CYLINDER, TYPES, COUNT>(sc.geoms(), r, ty, slot, prim, n_prims);
+    test_type<G_POLYHEDRON, TYPES, COUNT>(sc.geoms(), r, ty, slot, prim, n_prims);
+    test_type<G_MESH, TYPES, COUNT>(sc.geoms(), r, ty, slot, prim, n_prims);
+    test_type<G_POLYGON, TYPES, COUNT>(sc.geoms(), r, ty, slot, prim, n_prims);
+    }
+
+template<uint32_t TYPES, bool COUNT, bool UNI>
+__device__ __forceinline__ void search_leaf(const SearchScene<UNI>& sc, Search& r, uint32_t& n_prims)
+    {
+    if constexpr (TYPES == T_SPHERES)
+        search_sphere<COUNT, UNI>(sc, r, n_prims);
+    else
+        search_mixed<TYPES, COUNT, UNI>(sc, r, n_prims);
+    }
+
+template<uint32_t TYPES, bool UNI>
+__device__ __forceinline__ HitT search_end(const SearchScene<UNI>& sc, const Search& r)
+    {
+    HitT h = r.best;
+    if (TYPES == T_SPHERES && h.prim != EMPTY)
+        {
+        const uint2 id = ldg(sc.leaf_ref(), h.prim);
+        h.geom = id.x;
+        h.prim = id.y;
+        }
+    return h;
+    }
+
+// Closest hit of one ray per lane.  The wavefront visits nodes until the lanes
+// waiting at leaves are at least LEAF_WAIT times those still at inner nodes:
+// 1 for spheres (1/4, 1/2, 1, 2: 9.3, 9.1, 9.2, 9.3 ms of traversal on the
+// lattice of 1M spheres, 84M rays), 2 for the longer tests of other types
+// (1/2, 1, 2, 4: 12.5, 11.4, 10.9, 10.9 ms on the mixed scene of 1.8M
+// primitives, 14M rays).
+template<class Stack, bool COUNT, uint32_t TYPES, bool UNI>
+__device__ inline void trace_closest(const SceneDev& scene, v3 o, v3 d, float tnear, HitT& best, Stack& st,
+                                     uint32_t& n_nodes, uint32_t& n_prims, uint32_t& err)
+    {
+    constexpr uint32_t LEAF_WAIT = TYPES == T_SPHERES ? 1 : 2;
+    const SearchScene<UNI> sc(scene);
+    Search r;
+    search_begin(scene, o, d, tnear, r, st);
+    for (;;)
+        {
+        for (;;)
+            {
+            const bool inner = !(r.cur & LEAF);
+            const uint32_t n_in = (uint32_t)__popcll(__ballot(inner));
+            const uint32_t n_leaf = (uint32_t)__popcll(__ballot((r.cur & LEAF) && r.cur != EMPTY));
+            if (n_in == 0 || n_leaf >= LEAF_WAIT * n_in)
+                break;
+            if (inner)
+                search_visit<Stack, COUNT>(sc.nodes4(), r, st, n_nodes, err);
+            }
+        const bool leaf = (r.cur & LEAF) && r.cur != EMPTY;
+        if (__ballot(leaf) == 0)
+            break;
+        if (leaf)
+            {
+            search_leaf<TYPES, COUNT, UNI>(sc, r, n_prims);
+            search_pop(r, st);
+            }
+        }
+    best = search_end<TYPES, UNI>(sc, r);
     }
 
 // A ray queue is cut into QSEG segments with one append counter each, the
@@ -976,13 +1133,14 @@ struct Claims
         }
     };
 
-// The search is latency-bound (dependent node loads), so wavefronts in flight
-// matter: the spheres-only variant is held to 71 registers (7 wavefronts per
-// SIMD, no spills; 8 spill and run 7 % slower), the others to 64 (8 per SIMD,
-// a few values spill; on C3 the traversal takes 51 ms per frame at 8, 53 at
-// 7, 57 at 6 and 65 at the 5 its 87 registers allow).
+// Held to 72 registers (7 wavefronts per SIMD): at 6, 7, 8 the lattice of 1M
+// spheres takes 9.3, 9.2, 10.2 ms of traversal; at 5, 6, 7, 8 the mixed scene
+// takes 10.7, 10.0, 9.5, 10.9 ms and the mesh scene 9.7, 9.2, 9.2, 10.4 ms
+// (fewer wavefronts hide less of the node loads, at 8 values of the search
+// spill).  Before the 4-wide search of all scene types those scenes took
+// 11.4, 14.4 and 15.3 ms.
 template<int BLOCK, int SS, bool COUNT, bool PRIMARY, uint32_t TYPES>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == T_SPHERES ? 7 : 8))) void k_traverse(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_traverse(
     const JobDev* __restrict__ jobs, uint32_t n_jobs, Queue q, uint32_t n, const QueueView* __restrict__ view,
     uint4* hits, uint32_t* work, uint32_t chunk, uint32_t bands, uint2* gstack, uint32_t gstride,
     unsigned long long* counters)
@@ -1036,12 +1194,21 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == 
                 tnear = a.w;
                 job = __float_as_uint(b.w);
                 }
-            const SceneDev& sc = jobs[job].scene;
+            // one job at a time, so that the scene's pointers are scalar: nearly
+            // every wavefront's rays belong to one (the queues are filled chunk by
+            // chunk, a chunk's rays by one job)
             HitT h;
-            if constexpr (TYPES == T_SPHERES)
-                trace_closest<LdsStack<SS>, COUNT, TYPES>(sc, o, d, tnear, h, st, n_nodes, n_prims, err);
-            else
-                trace_closest_grouped<LdsStack<SS>, COUNT, TYPES>(sc, o, d, tnear, h, st, n_nodes, n_prims, err);
+            for (bool todo = true; __ballot(todo) != 0;)
+                if (todo)
+                    {
+                    const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)job);
+                    if (job == j0)
+                        {
+                        trace_closest<LdsStack<SS>, COUNT, TYPES, true>(jobs[j0].scene, o, d, tnear, h, st, n_nodes,
+                                                                        n_prims, err);
+                        todo = false;
+                        }
+                    }
             hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, 0);
             if (COUNT)
                 n_rays++;
@@ -1340,8 +1507,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(LOOP ? 7 : 1
 // only on nodes it wants (its own slab and cull tests passed at the parent),
 // so each ray's result is the one the per-ray search returns; the wavefront
 // descends into a child when any lane wants it, nearer child first by lane
-// majority, and pushes the other with each lane's own cull bound.  Groups of
-// 64 rays that straddle two jobs fall back to the per-ray search.
+// majority, and pushes the other with each lane's own cull bound.  A group of
+// 64 rays that straddles jobs is searched once for each.
 constexpr uint32_t UNWANTED = 0x80000000u; // stack flag: this lane does not need the node
 typedef const float __attribute__((address_space(4))) ConstF;
 typedef const uint32_t __attribute__((address_space(4))) ConstU;
@@ -1377,35 +1544,38 @@ struct EntryCount
 
 // Closest hits of one wavefront's 64 primary rays (lane ray o, d of job `job`
 // at pixel px, py; `valid` lanes only): tile lists when all 64 rays form one
-// full tile of a job that has them, wavefront-packet BVH search when they
-// belong to one job, per-ray search otherwise.
-template<int SS, bool COUNT, uint32_t TYPES>
+// full tile of a job that has them, else a wavefront-packet BVH search for
+// each job.  ONE_JOB: every lane's job is the same (a scalar).
+template<int SS, bool COUNT, uint32_t TYPES, bool ONE_JOB>
 __device__ __forceinline__ void primary_group_hit(const JobDev* __restrict__ jobs, bool valid, uint32_t job,
                                                   uint32_t px, uint32_t py, v3 o, v3 d, float tnear,
                                                   LdsStack<SS>& st, HitT& best, uint32_t& n_nodes,
                                                   uint32_t& n_prims, EntryCount& n_entries, uint32_t& err)
     {
-    const uint32_t job0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)job);
-    const bool one_job = __ballot(valid && job != job0) == 0;
+    // one job at a time (nearly always all 64 rays belong to one)
+    uint64_t left = __ballot(valid);
+    if (left == 0)
+        return;
+    do
+    {
+    const uint32_t first = ONE_JOB ? 0u : (uint32_t)(__ffsll((unsigned long long)left) - 1);
+    const uint32_t job0 = (uint32_t)__builtin_amdgcn_readlane((int)job, first);
+    const bool mine = ONE_JOB ? valid : (valid && job == job0);
+    const uint64_t m_mine = __ballot(mine);
+    left &= ~m_mine;
     // the tile of this group, if all 64 rays belong to one full 8x8 tile
     uint32_t tile = EMPTY;
-    if (one_job && jobs[job0].use_tiles)
+    if (m_mine == ~0ull && jobs[job0].use_tiles)
         {
         const JobDev& J = jobs[job0];
-        if (valid && px < J.tiles_x * TILE && py < J.tiles_y * TILE)
+        if (px < J.tiles_x * TILE && py < J.tiles_y * TILE)
             tile = (py / TILE) * J.tiles_x + px / TILE;
         const uint32_t t0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)tile);
         if (__ballot(tile != t0) != 0)
             tile = EMPTY;
         tile = (uint32_t)__builtin_amdgcn_readfirstlane((int)tile);
         }
-    if (!one_job)
-        {
-        if (valid)
-            trace_closest<LdsStack<SS>, COUNT, TYPES>(jobs[job].scene, o, d, tnear, best, st, n_nodes,
-                                                      n_prims, err);
-        }
-    else if (tile != EMPTY)
+    if (tile != EMPTY)
         {
         // candidate list of the tile (kernels/tiles.hip), nearest bound
         // first; the next entry is loaded while the current one is tested
@@ -1505,7 +1675,6 @@ __device__ __forceinline__ void primary_group_hit(const JobDev* __restrict__ job
                                 ts.margin = J.scene.cull_margin;
                                 ts.best = best;
                                 ts.node = r & ~NODE_REF;
-                                ts.sph = false;
                                 st.sp = 0;
                                 while (trace_visit2<LdsStack<SS>, COUNT, TYPES>(J.scene.nodes, geoms, ts, st, n_nodes,
                                                                                 n_prims, err))
@@ -1545,12 +1714,15 @@ __device__ __forceinline__ void primary_group_hit(const JobDev* __restrict__ job
         const GeomDev* __restrict__ geoms = sc.geoms;
         const v3 inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
         const float margin = sc.cull_margin;
-        best.t = __builtin_huge_valf();
-        best.geom = EMPTY;
-        best.prim = EMPTY;
+        if (mine)
+            {
+            best.t = __builtin_huge_valf();
+            best.geom = EMPTY;
+            best.prim = EMPTY;
+            }
         st.sp = 0;
         uint32_t node = sc.root;
-        bool want = valid;
+        bool want = mine;
         while (node != EMPTY)
             {
             // the node index is uniform: fetch through the constant address
@@ -1648,6 +1820,7 @@ __device__ __forceinline__ void primary_group_hit(const JobDev* __restrict__ job
                 }
             }
         }
+    } while (!ONE_JOB && left != 0);
     }
 
 template<int BLOCK, int SS, bool COUNT, uint32_t TYPES>
@@ -1689,7 +1862,7 @@ __global__ __launch_bounds__(BLOCK) void k_traverse_packet(const JobDev* __restr
                 primary_ray(jobs, n_jobs, i, job, k, px, py, jord, o, d);
                 }
             HitT best;
-            primary_group_hit<SS, COUNT, TYPES>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes, n_prims,
+            primary_group_hit<SS, COUNT, TYPES, false>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes, n_prims,
                                                 n_entries, err);
             if (valid)
                 {
@@ -1764,20 +1937,20 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == 
         const uint32_t u = bands ? (c % QSEG) * G + c / QSEG : c;
         const uint32_t seg = bands ? u / G : u % QSEG; // the chunk's output segment
         const uint32_t base = u * chunk;
-        // one job for the whole chunk (every chunk of a single-job batch, all
-        // but the chunks that straddle two jobs otherwise): its index is
-        // workgroup-uniform, so the job record arrives by scalar loads; the
-        // branch is taken by the whole workgroup, barriers included
+        // the chunk's jobs one after the other (one, unless it straddles two):
+        // the job's index is workgroup-uniform, so its record arrives by scalar
+        // loads and the loop is taken by the whole workgroup, barriers included
         const uint32_t last = min(n, base + chunk) - 1u;
         const uint32_t job_first = (uint32_t)__builtin_amdgcn_readfirstlane((int)find_job(jobs, n_jobs, base));
         const uint32_t job_last = (uint32_t)__builtin_amdgcn_readfirstlane((int)find_job(jobs, n_jobs, last));
-        if (u < n_units && job_first == job_last)
+        for (uint32_t job = job_first; job <= job_last && u < n_units; job++)
             {
-            const JobDev& J = jobs[job_first];
+            const JobDev& J = jobs[job];
+            const uint32_t end = (job == job_last) ? n : jobs[job + 1].ray_base;
             for (uint32_t g = 0; g < groups; g++)
                 {
                 const uint32_t i = base + (wave * groups + g) * 64 + lane;
-                const bool valid = i < n;
+                const bool valid = i >= J.ray_base && i < end;
                 v3 o = mk3(0.0f, 0.0f, 0.0f), d = mk3(0.0f, 0.0f, 1.0f);
                 uint32_t k = 0, px = 0, py = 0, jord = 0;
                 if (valid)
@@ -1786,34 +1959,14 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == 
                 best.t = __builtin_huge_valf();
                 best.geom = EMPTY;
                 best.prim = EMPTY;
-                primary_group_hit<SS, COUNT, TYPES>(jobs, valid, job_first, px, py, o, d, 1e-3f, st, best, n_nodes,
-                                                    n_prims, n_entries, err);
+                primary_group_hit<SS, COUNT, TYPES, true>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes,
+                                                          n_prims, n_entries, err);
                 if (COUNT && valid)
                     n_rays++;
-                shade_primary_block<BLOCK, TYPES>(jobs, valid, job_first, k, py * J.W + px, jord, o, d, best, out,
-                                                  seg, records, sh);
+                shade_primary_block<BLOCK, TYPES>(jobs, valid, job, k, py * J.W + px, jord, o, d, best, out, seg,
+                                                  records, sh);
                 }
             }
-        else
-            for (uint32_t g = 0; g < groups && u < n_units; g++)
-                {
-                const uint32_t i = base + (wave * groups + g) * 64 + lane;
-                const bool valid = i < n;
-                v3 o = mk3(0.0f, 0.0f, 0.0f), d = mk3(0.0f, 0.0f, 1.0f);
-                uint32_t job = 0, k = 0, px = 0, py = 0, jord = 0;
-                if (valid)
-                    primary_ray(jobs, n_jobs, i, job, k, px, py, jord, o, d);
-                HitT best;
-                best.t = __builtin_huge_valf();
-                best.geom = EMPTY;
-                best.prim = EMPTY;
-                primary_group_hit<SS, COUNT, TYPES>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes,
-                                                    n_prims, n_entries, err);
-                if (COUNT && valid)
-                    n_rays++;
-                shade_primary_block<BLOCK, TYPES>(jobs, valid, job, k, py * jobs[job].W + px, jord, o, d, best, out,
-                                                  seg, records, sh);
-                }
         __syncthreads();
         c = s_claim;
         __syncthreads();
@@ -1882,7 +2035,7 @@ __global__ __launch_bounds__(BLOCK) void k_bounce(const JobDev* __restrict__ job
                 const float4 at4 = in.att[sl];
                 const v3 o = mk3(a.x, a.y, a.z), d = mk3(b.x, b.y, b.z);
                 HitT h;
-                trace_closest<LdsStack<SS>, COUNT, TYPES>(J.scene, o, d, a.w, h, st, n_nodes, n_prims, err);
+                trace_closest<LdsStack<SS>, COUNT, TYPES, false>(J.scene, o, d, a.w, h, st, n_nodes, n_prims, err);
                 if (COUNT)
                     n_rays++;
                 att = mk3(at4.x, at4.y, at4.z);
@@ -1996,10 +2149,8 @@ __global__ __launch_bounds__(BLOCK) void k_traverse_dyn(const JobDev* __restrict
     prefetch();
     bool active = false;
     uint32_t i = 0;
-    TraceState r;
-    const Node* nodes2 = nullptr;
-    const Node4* nodes4 = nullptr;
-    const GeomDev* geoms = nullptr;
+    Search r;
+    uint32_t job = 0;
     for (;;)
         {
         const uint32_t n_idle = (uint32_t)__popcll(__ballot(!active));
@@ -2012,7 +2163,6 @@ __global__ __launch_bounds__(BLOCK) void k_traverse_dyn(const JobDev* __restrict
                 pf = EMPTY;
                 v3 o, d;
                 float tnear;
-                uint32_t job;
                 if (PRIMARY)
                     {
                     uint32_t k, pixel, jord;
@@ -2026,28 +2176,28 @@ __global__ __launch_bounds__(BLOCK) void k_traverse_dyn(const JobDev* __restrict
                     tnear = pa.w;
                     job = __float_as_uint(pb.w);
                     }
-                const SceneDev& sc = jobs[job].scene;
-                nodes2 = sc.nodes;
-                nodes4 = sc.nodes4;
-                geoms = sc.geoms;
-                trace_begin(sc, o, d, tnear, r, st);
+                search_begin(jobs[job].scene, o, d, tnear, r, st);
                 active = true;
                 }
             prefetch();
             }
         if (__ballot(active) == 0)
             break;
-        bool more = false;
         if (active)
             {
-            if constexpr (TYPES == T_SPHERES)
-                more = trace_visit4<LdsStack<SS>, COUNT, TYPES>(nodes4, geoms, r, st, n_nodes, n_prims, err);
-            else
-                more = trace_visit2<LdsStack<SS>, COUNT, TYPES>(nodes2, geoms, r, st, n_nodes, n_prims, err);
+            const SearchScene<false> sc(jobs[job].scene);
+            if (!(r.cur & LEAF))
+                search_visit<LdsStack<SS>, COUNT>(sc.nodes4(), r, st, n_nodes, err);
+            else if (r.cur != EMPTY)
+                {
+                search_leaf<TYPES, COUNT, false>(sc, r, n_prims);
+                search_pop(r, st);
+                }
             }
-        if (active && !more)
+        if (active && r.cur == EMPTY)
             {
-            hits[i] = make_uint4(__float_as_uint(r.best.t), r.best.geom, r.best.prim, 0);
+            const HitT h = search_end<TYPES, false>(jobs[job].scene, r);
+            hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, 0);
             active = false;
             if (COUNT)
                 n_rays++;
@@ -2065,7 +2215,7 @@ __global__ __launch_bounds__(BLOCK) void k_traverse_dyn(const JobDev* __restrict
     }
 
 // Tail: each thread finishes its path (trace + shade until termination).
-template<int SS, bool COUNT, uint32_t TYPES>
+template<int SS, bool COUNT, uint32_t TYPES, bool UNI>
 __device__ __forceinline__ void finish_path(const JobDev& J, const uint4& mt, v3 o, v3 d, v3 att, LdsStack<SS>& st,
                                             uint4* records, uint32_t max_depth, unsigned long long* counters,
                                             uint32_t& n_nodes, uint32_t& n_prims, uint32_t& n_rays, uint32_t& err)
@@ -2076,10 +2226,7 @@ __device__ __forceinline__ void finish_path(const JobDev& J, const uint4& mt, v3
     for (;;)
         {
         HitT h;
-        if constexpr (TYPES == T_SPHERES)
-            trace_closest<LdsStack<SS>, COUNT, TYPES>(J.scene, o, d, 1e-3f, h, st, n_nodes, n_prims, err);
-        else
-            trace_closest_grouped<LdsStack<SS>, COUNT, TYPES>(J.scene, o, d, 1e-3f, h, st, n_nodes, n_prims, err);
+        trace_closest<LdsStack<SS>, COUNT, TYPES, UNI>(J.scene, o, d, 1e-3f, h, st, n_nodes, n_prims, err);
         if (COUNT)
             n_rays++;
         v3 no, nd;
@@ -2130,10 +2277,10 @@ __global__ __launch_bounds__(BLOCK) void k_finish(const JobDev* __restrict__ job
         const v3 o = mk3(a.x, a.y, a.z), d = mk3(b.x, b.y, b.z), att = mk3(at4.x, at4.y, at4.z);
         const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)mt.x);
         if (n_jobs == 1 || __ballot(mt.x != j0) == 0)
-            finish_path<SS, COUNT, TYPES>(jobs[j0], mt, o, d, att, st, records, max_depth, counters, n_nodes,
+            finish_path<SS, COUNT, TYPES, true>(jobs[j0], mt, o, d, att, st, records, max_depth, counters, n_nodes,
                                           n_prims, n_rays, err);
         else
-            finish_path<SS, COUNT, TYPES>(jobs[mt.x], mt, o, d, att, st, records, max_depth, counters, n_nodes,
+            finish_path<SS, COUNT, TYPES, false>(jobs[mt.x], mt, o, d, att, st, records, max_depth, counters, n_nodes,
                                           n_prims, n_rays, err);
         }
     if (COUNT)
@@ -2289,14 +2436,19 @@ __device__ __forceinline__ float4 preview_shade(const JobDev& J, const HitT& h, 
 // LDS, where one thread per pixel and channel adds them in sample order (the
 // order of the reference's loop, so the sum does not depend on the split).
 // Otherwise (fewer samples than wavefronts) each wavefront has a chunk to
-// itself.  The kernel is bound by VALU issue (camera rays with Philox, the
+// itself.  own_search: each lane searches the binary hierarchy for its own ray
+// (scenes with convex polyhedra: a face nearly parallel to a ray gives a
+// computed distance up to units below its box's entry, so which hit is found
+// first decides, and the order stays that of the search per ray).
+// The kernel is bound by VALU issue (camera rays with Philox, the
 // lights' acos, sin and cos).  One pixel per thread with its own search and
 // 64 serial samples, in raster order with the stack in scratch, took 5.99 ms
-// for 500 spheres at 600 x 370 and 36.7 ms for 20,000 polyhedra at 1280 x
-// 720, 64 samples each, image read included; this form takes 0.67 and 6.4 ms.
+// for 500 spheres at 600 x 370 and 34.3 ms for 20,000 polyhedra at 1280 x
+// 720, 64 samples each, image read included; this form takes 0.67 and 16.8 ms.
 template<int BLOCK, int SS, uint32_t TYPES, bool SPLIT>
-__global__ __launch_bounds__(BLOCK) void k_preview(const JobDev* __restrict__ jobp, uint32_t aa_n, uint2* gstack,
-                                                   uint32_t gstride, unsigned long long* counters)
+__global__ __launch_bounds__(BLOCK) void k_preview(const JobDev* __restrict__ jobp, uint32_t aa_n,
+                                                   uint32_t own_search, uint2* gstack, uint32_t gstride,
+                                                   unsigned long long* counters)
     {
     constexpr uint32_t WAVES = BLOCK / 64;
     static_assert(BLOCK == 256, "one thread per pixel and channel of a chunk");
@@ -2340,8 +2492,14 @@ __global__ __launch_bounds__(BLOCK) void k_preview(const JobDev* __restrict__ jo
                 h.t = __builtin_huge_valf();
                 h.geom = EMPTY;
                 h.prim = EMPTY;
-                primary_group_hit<SS, false, TYPES>(jobp, valid, 0, px, py, o, d, 0.0f, st, h, n_nodes, n_prims,
-                                                    n_entries, err);
+                if (TYPES != T_SPHERES && own_search)
+                    {
+                    if (valid)
+                        trace_binary<LdsStack<SS>, false, TYPES>(J.scene, o, d, 0.0f, h, st, n_nodes, n_prims, err);
+                    }
+                else
+                    primary_group_hit<SS, false, TYPES, true>(jobp, valid, 0, px, py, o, d, 0.0f, st, h, n_nodes,
+                                                              n_prims, n_entries, err);
                 if (valid)
                     c = preview_shade<TYPES>(J, h, o, d);
                 }
@@ -2429,6 +2587,7 @@ __global__ void k_debug_sincos(const float* x, uint32_t n, float* s, float* c)
     }
 
 // Primary ray and closest hit per pixel for camera sample `sample`.
+template<uint32_t TYPES>
 __global__ void k_debug_primary(const JobDev* __restrict__ jobp, uint32_t sample, float* rays, uint4* hits)
     {
     const JobDev& J = *jobp;
@@ -2441,7 +2600,7 @@ __global__ void k_debug_primary(const JobDev* __restrict__ jobp, uint32_t sample
     LocalStack st;
     uint32_t dummy = 0, err = 0;
     HitT h;
-    trace_closest<LocalStack, false>(J.scene, o, d, 1e-3f, h, st, dummy, dummy, err);
+    trace_closest<LocalStack, false, TYPES, true>(J.scene, o, d, 1e-3f, h, st, dummy, dummy, err);
     float* r = rays + 6 * (size_t)pixel;
     r[0] = o.x;
     r[1] = o.y;
@@ -2452,6 +2611,7 @@ __global__ void k_debug_primary(const JobDev* __restrict__ jobp, uint32_t sample
     hits[pixel] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, err);
     }
 
+template<uint32_t TYPES>
 __global__ void k_debug_trace(const SceneDev sc, const float* rays, uint32_t n, float tnear, uint4* hits)
     {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2461,7 +2621,7 @@ __global__ void k_debug_trace(const SceneDev sc, const float* rays, uint32_t n, 
     LocalStack st;
     uint32_t dummy = 0, err = 0;
     HitT h;
-    trace_closest<LocalStack, false>(sc, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), tnear, h, st, dummy, dummy,
+    trace_closest<LocalStack, false, TYPES, true>(sc, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), tnear, h, st, dummy, dummy,
                                      err);
     hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, err);
     }

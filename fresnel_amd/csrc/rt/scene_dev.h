@@ -82,19 +82,18 @@ struct __attribute__((aligned(64))) Node
     uint4 link;   // c0, c1, g0, g1
     };
 
-// 4-wide node (128 bytes): two child pairs, each laid out as a binary node
-// (children 2p and 2p + 1 of pair p: boxes, references, geometry slots), so a
-// search step loads and tests one pair at a time.  A child reference is a
-// 4-wide node index, LEAF | local primitive index (geometry slot alongside)
-// or EMPTY with a NaN box.  In a spheres-only scene (SceneDev::sphere_leaves)
-// every child holds a centre c in lo.xyz and half extents h in hi.xyz, and its
-// box is c -+ h: a leaf child its sphere (h = radius on every axis, so the box
-// is exactly the builder's bounds), an inner child a box that contains the
-// exact one after rounding.
-struct __attribute__((aligned(128))) Node4
+// 4-wide node (64 bytes): on each axis child k's box is
+// [o + s * lo_k, o + s * hi_k], lo_k and hi_k byte k of qlo and qhi, rounded
+// outwards and padded against the rounding of the search's slab test
+// (NODE_PAD, k_bvh4_fill); its reference is a 4-wide node index, LEAF | the
+// leaf's position in the hierarchy's leaf order, or EMPTY (children 2 and 3).
+struct __attribute__((aligned(64))) Node4
     {
-    Node pair[2];
+    float o[3], s[3];
+    uint32_t qlo[3], qhi[3];
+    uint32_t ref[4];
     };
+constexpr float NODE_PAD = 0x1p-20f;
 
 struct SceneDev
     {
@@ -102,10 +101,15 @@ struct SceneDev
     const Node4* nodes4; // root: node 0 (as for nodes) unless root is EMPTY
     const GeomDev* geoms;
     uint32_t root;      // EMPTY when the scene has no primitive
-    uint32_t sphere_leaves; // 4-wide leaf children hold spheres (spheres-only scene)
+    uint32_t sphere_leaves; // leaf holds spheres (spheres-only scene)
     uint32_t n_geoms;
     uint32_t n_prims;
     float cull_margin;  // CULL_K * 3 * largest primitive half-extent
+    // leaf data in leaf order: spheres-only, (x, y, z, r) and the geometry slot
+    // and primitive beside it in leaf_ref; otherwise two per leaf, the bounds
+    // lo.xyz | slot, hi.xyz | primitive
+    const float4* leaf;
+    const uint2* leaf_ref;
     };
 
 // Camera constants derived on the host from the UserCamera

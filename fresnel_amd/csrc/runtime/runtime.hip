@@ -686,7 +686,9 @@ struct SceneObj
     bool build_pending = false;  // a build or refit was queued on the device stream since its last sync
     DBuf<Node> nodes;
     DBuf<Node4> nodes4;
-    bool sphere_leaves = false; // nodes4 leaf children hold spheres
+    bool sphere_leaves = false; // leaf holds spheres (else bounds)
+    DBuf<float4> leaf;          // leaf data in leaf order (SceneDev::leaf)
+    DBuf<uint2> leaf_ref;
     DBuf<uint32_t> idx4; // 4-wide node of each binary inner node (exclusive scan of even-depth flags)
     uint32_t n_prims = 0;
     uint32_t n_active = 0; // geometries with primitives: entries of prefix / slots
@@ -999,6 +1001,9 @@ static void build_bvh(SceneObj& sc, bool refit_only)
     }
     sc.nodes.ensure(std::max<uint32_t>(N - 1, 1));
     sc.root_box.ensure(6);
+    sc.leaf.ensure(sc.sphere_leaves ? N : 2 * (size_t)N);
+    sc.leaf_ref.ensure(sc.sphere_leaves ? N : 1);
+    const GeomDev* sphere_geoms = sc.sphere_leaves ? sc.dgeoms.p : nullptr;
     if (N == 1)
         {
         static const uint32_t one[2] = {0u, 1u};
@@ -1008,9 +1013,9 @@ static void build_bvh(SceneObj& sc, bool refit_only)
         D.launch("lbvh_single",
                  [&]
                  {
-                     k_single_leaf<<<1, 1, 0, s>>>(sc.blo.p, sc.bhi.p, sc.nodes.p);
-                     k_bvh4_fill<<<1, 64, 0, s>>>(sc.nodes.p, 1, sc.idx4.p, sc.nodes4.p,
-                                                   sc.sphere_leaves ? sc.dgeoms.p : nullptr);
+                     k_single_leaf<<<1, 1, 0, s>>>(sc.blo.p, sc.bhi.p, sc.nodes.p, sphere_geoms, sc.leaf.p,
+                                                   sc.leaf_ref.p);
+                     k_bvh4_fill<<<1, 64, 0, s>>>(sc.nodes.p, 1, sc.idx4.p, nullptr, sc.nodes4.p);
                  });
         sc.bvh_valid = true;
         sc.builds++;
@@ -1064,13 +1069,14 @@ static void build_bvh(SceneObj& sc, bool refit_only)
              [&]
              {
                  k_refit<<<blocks(N, 256), 256, 0, s>>>(sc.vals.p, sc.blo.p, sc.bhi.p, (int)N, sc.nodes.p,
-                                                        sc.parent.p, sc.flags.p, sc.root_box.p);
+                                                        sc.parent.p, sc.flags.p, sc.root_box.p, sphere_geoms,
+                                                        sc.leaf.p, sc.leaf_ref.p);
              });
     D.launch("lbvh_bvh4",
              [&]
              {
-                 k_bvh4_fill<<<blocks(N - 1, 256), 256, 0, s>>>(sc.nodes.p, N - 1, sc.idx4.p, sc.nodes4.p,
-                                                                 sc.sphere_leaves ? sc.dgeoms.p : nullptr);
+                 k_bvh4_fill<<<blocks(N - 1, 256), 256, 0, s>>>(sc.nodes.p, N - 1, sc.idx4.p, sc.parent.p,
+                                                                 sc.nodes4.p);
              });
     sc.bvh_valid = true;
     }
@@ -1201,6 +1207,8 @@ static SceneDev scene_dev(SceneObj& sc)
     d.n_geoms = sc.n_slots;
     d.n_prims = sc.n_prims;
     d.cull_margin = sc.cull_margin;
+    d.leaf = sc.leaf.p;
+    d.leaf_ref = sc.leaf_ref.p;
     return d;
     }
 
@@ -1680,8 +1688,8 @@ struct BatchExec
             }
         REQUIRE(n_pri < (1ull << 31) && n_paths < (1ull << 31), "batch too large");
         for (const auto& J : jobs)
-            REQUIRE(!spheres || J.scene.sphere_leaves || J.scene.root == EMPTY,
-                    "internal error: spheres-only kernels on a hierarchy without sphere leaves");
+            REQUIRE(J.scene.root == EMPTY || spheres == (J.scene.sphere_leaves != 0),
+                    "internal error: spheres-only kernels and a hierarchy with sphere leaves go together");
         // primary rays are generated from their index; the queues hold paths
         uint32_t max_l = 1;
         for (const auto& J : jobs)
@@ -2238,7 +2246,9 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     // direct tracers do not support depth of field (fresnel/cpu/TracerDirect.cc:38-40)
     fh_user_camera cam = sc.camera;
     cam.f_stop = __builtin_huge_valf();
-    update_tiles(D, sc, tr, make_cam(cam), (uint64_t)tr.W * tr.H * tr.aa_n * tr.aa_n);
+    const bool own_search = (scene_types(sc) & (1u << G_POLYHEDRON)) != 0;
+    if (!own_search)
+        update_tiles(D, sc, tr, make_cam(cam), (uint64_t)tr.W * tr.H * tr.aa_n * tr.aa_n);
     JobDev J = make_job(sc, tr, cam);
     J.K = 1;
     set_order_divisors(J);
@@ -2258,7 +2268,8 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     const uint32_t gstride = grid * PREVIEW_BLOCK;
     R.gstack.ensure((size_t)(STACK_MAX - 8) * gstride);
     D.launch("preview",
-             [&] { kern<<<grid, PREVIEW_BLOCK, 0, D.stream>>>(R.jobs.p, tr.aa_n, R.gstack.p, gstride, D.counters.p); });
+             [&] { kern<<<grid, PREVIEW_BLOCK, 0, D.stream>>>(R.jobs.p, tr.aa_n, own_search ? 1u : 0u, R.gstack.p,
+                                                         gstride, D.counters.p); });
     D.end_stats();
     if (D.last_counters[CTR_OVERFLOW])
         throw Error(FH_ERR_STATE, "traversal stack overflow");
@@ -4310,7 +4321,8 @@ extern "C"
                 DBuf<uint4> dhits;
                 dhits.ensure(npix);
                 HIPCHECK(hipMemcpy(dj.p, &J, sizeof(J), hipMemcpyHostToDevice));
-                k_debug_primary<<<blocks(npix, 64), 64, 0, D.stream>>>(dj.p, sample, drays.p, dhits.p);
+                auto* kern = scene->obj.sphere_leaves ? k_debug_primary<T_SPHERES> : k_debug_primary<T_ALL>;
+                kern<<<blocks(npix, 64), 64, 0, D.stream>>>(dj.p, sample, drays.p, dhits.p);
                 HIPCHECK(hipGetLastError());
                 HIPCHECK(hipStreamSynchronize(D.stream));
                 std::vector<uint4> h(npix);
@@ -4363,7 +4375,7 @@ extern "C"
                 TravArgs a {R.jobs.p, 1, Queue {}, npix, nullptr, R.hits.p, R.counters32.p, D.trav_chunk, R.gstack.p,
                             gstride, D.counters.p};
                 dispatch_traverse(D, "traverse_primary", D.stream, a, true,
-                                  (scene_types(sc) & ~T_SPHERES) == 0);
+                                  sc.sphere_leaves);
                 D.end_stats();
                 if (D.last_counters[CTR_OVERFLOW])
                     throw Error(FH_ERR_STATE, "traversal stack overflow");
@@ -4440,7 +4452,8 @@ extern "C"
                 DBuf<uint4> dhits;
                 dhits.ensure(n);
                 HIPCHECK(hipMemcpy(drays.p, rays, 24 * (size_t)n, hipMemcpyHostToDevice));
-                k_debug_trace<<<blocks(n, 64), 64, 0, D.stream>>>(scene_dev(scene->obj), drays.p, n, tnear, dhits.p);
+                auto* kern = scene->obj.sphere_leaves ? k_debug_trace<T_SPHERES> : k_debug_trace<T_ALL>;
+                kern<<<blocks(n, 64), 64, 0, D.stream>>>(scene_dev(scene->obj), drays.p, n, tnear, dhits.p);
                 HIPCHECK(hipGetLastError());
                 HIPCHECK(hipStreamSynchronize(D.stream));
                 std::vector<uint4> h(n);

@@ -1,0 +1,91 @@
+"""The 4-wide search against brute force: directions with zero and tiny components, flat and tiny scenes, few primitives."""
+
+import ctypes
+
+import numpy
+import pytest
+
+import fresnel_amd as fresnel
+import oracle
+from oracle import ptr
+import scenes
+from test_gpu_parity import c1_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def spheres(n, scale, offset=0.0, radius=0.5):
+    def build(device):
+        rng = numpy.random.default_rng(n)
+        s = fresnel.Scene(device)
+        pos = rng.uniform(-2, 2, (n, 3)) * scale + offset
+        fresnel.geometry.Sphere(s, position=pos.astype(numpy.float32), radius=radius * scale)
+        return s
+    return build
+
+
+def flat(device):
+    """Triangles in the planes x = 0, y = 0 and z = 3, polygons in z = 0, spherocylinders along the axes."""
+    s = fresnel.Scene(device)
+    tri = [[0, -1, -1], [0, 1, -1], [0, -1, 1], [-1, 0, -1], [1, 0, -1], [-1, 0, 1], [-1, -1, 3], [1, -1, 3], [-1, 1, 3]]
+    fresnel.geometry.Mesh(s, tri, position=[[0, 0, 0], [0, 0, 2], [3, 0, 0]], orientation=[[1, 0, 0, 0]] * 3)
+    fresnel.geometry.Polygon(s, [[-1, -1], [1, -1], [0, 1]], position=[[0, 0], [2, 1], [-2, 0]], angle=[0, 0.5, 1])
+    fresnel.geometry.Cylinder(s, points=[[[0, 0, 0], [2, 0, 0]], [[0, 0, 0], [0, 0, -2]], [[0, 1, 0], [0, 1, 0]]],
+                              radius=0.1)
+    return s
+
+
+SCENES = {
+    'spheres_1': spheres(1, 1.0),
+    'spheres_2': spheres(2, 1.0),
+    'spheres_3': spheres(3, 1.0),
+    'spheres_5': spheres(5, 1.0),
+    'spheres_700': spheres(700, 8.0, radius=0.02),
+    'spheres_milli': spheres(200, 1e-3),
+    'spheres_mega': spheres(200, 1e6),
+    'spheres_aside': spheres(200, 1.0, offset=1000.0),
+    'c1': c1_scene,
+    'flat': flat,
+    'polyhedra': scenes.eight_polyhedra,
+    'cylinders': scenes.four_cylinders,
+    'box': scenes.box,
+    'triangle': scenes.one_triangle,
+    'polygons': scenes.rounded_polygons,
+}
+
+
+def rays_of(scene, n, rng):
+    """Rays between and along box faces of the scene: all, one or two direction components zero or tiny."""
+    ext = scene.get_extents().astype(numpy.float64)
+    c, half = (ext[0] + ext[1]) / 2, numpy.maximum((ext[1] - ext[0]) / 2, 0.2 * (ext[1] - ext[0]).max())
+    o = c + rng.uniform(-2, 2, (n, 3)) * half
+    d = rng.normal(size=(n, 3))
+    small = [0.0, -0.0, 1e-45, 2.0**-61, -2.0**-60, 2.0**-59, 1e-12, -1e-6]
+    k = rng.integers(0, 4, n)  # 0: as it is, 1: one component small, 2: two, 3: two, and the origin on the scene's planes
+    axis = rng.integers(0, 3, n)
+    for i in range(n):
+        for j in range(3):
+            if (k[i] == 1 and j == axis[i]) or (k[i] >= 2 and j != axis[i]):
+                d[i, j] = small[rng.integers(len(small))]
+                if k[i] == 3:
+                    o[i, j] = [0.0, ext[0, j], ext[1, j], c[j]][rng.integers(4)]
+    d /= numpy.linalg.norm(d, axis=1, keepdims=True)
+    return numpy.ascontiguousarray(numpy.concatenate([o, d], axis=1), dtype=numpy.float32)
+
+
+@pytest.mark.parametrize('tnear', [0.0, 1e-3])
+@pytest.mark.parametrize('name', sorted(SCENES))
+def test_search_equals_brute_force(name, tnear, gpu_device, cpu_device):
+    """Geometry, primitive and distance of every ray are the brute-force minimum's, bit for bit."""
+    gs, cs = SCENES[name](gpu_device), SCENES[name](cpu_device)
+    n = 3000
+    rays = rays_of(cs, n, numpy.random.default_rng(5))
+    gid, prim, t = gs._scene.debugTrace(rays, tnear)
+    L, h = oracle.lib(), cs._scene.handle()
+    L.oracle_scene_set_brute(h, 1)
+    rg, rp, rt = numpy.zeros(n, numpy.uint32), numpy.zeros(n, numpy.uint32), numpy.zeros(n, numpy.float32)
+    L.oracle_trace(h, ptr(rays), n, tnear, ptr(rg, ctypes.c_uint32), ptr(rp, ctypes.c_uint32), ptr(rt), None, 0)
+    assert numpy.array_equal(gid, rg)
+    assert numpy.array_equal(prim, rp)
+    assert numpy.array_equal(t.view(numpy.uint32), rt.view(numpy.uint32))
+    assert (rg != 0xffffffff).any()
