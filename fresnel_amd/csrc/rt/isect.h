@@ -338,6 +338,24 @@ __device__ __forceinline__ GeomDev uniform_geom(const GeomDev* geoms, uint32_t s
     return g;
     }
 
+// x / d as (float)(x * inv) with inv = 1 / d in double (d float): the correctly
+// rounded float quotient.  A quotient of two floats lies at least 2^-49
+// (relative) from every midpoint of floats: x = m d for a midpoint m (25 bits)
+// would need x of more than 24 bits, so |x - m d| is at least one unit in the
+// last place of a 49-bit product.  The double reciprocal and product err by at
+// most 2^-52.  A quotient below 2^-126 (rounded to a multiple of 2^-149) may
+// differ by one such step; zero, infinite and NaN operands give IEEE results
+// (0 * inf and inf * 0 are NaN as 0 / 0 and inf / inf are).
+__device__ __forceinline__ float div_by(float x, double inv)
+    {
+    return (float)((double)x * inv);
+    }
+// The double whose words are (lo, hi).
+__device__ __forceinline__ double edge_rcp(float lo, float hi)
+    {
+    return __hiloint2double(__float_as_int(hi), __float_as_int(lo));
+    }
+
 // ---------------------------------------------------------------- intersect one primitive
 // The callbacks of fresnel/cpu/Geometry*.cc with `t < tfar` left to the caller.
 // Geometry-type sets a kernel is compiled for: a spheres-only scene uses
@@ -571,14 +589,18 @@ __device__ inline bool intersect_prim(const GeomDev& g, uint32_t prim, v3 o, v3 
         v2 p2;
         p2.x = rh.x;
         p2.y = rh.y;
-        // even-odd test with distance to the nearest edge (GeometryPolygon.cc:116-142)
+        // even-odd test with distance to the nearest edge (GeometryPolygon.cc:116-142).
+        // The two quotients by edge constants multiply by double reciprocals
+        // (div_by), and the square root is taken once, of the smallest squared
+        // distance: it rounds monotonically, so it is the smallest root.
         const uint32_t nv = g.n_aux;
-        float min_d = 3.40282346638528859812e+38f;
+        float min_sq = __builtin_huge_valf();
         bool odd = false;
         uint32_t j = nv - 1;
         for (uint32_t i = 0; i < nv; i++)
             {
             const float4 fi = ld4<UNI>(g.aux0, i), fj = ld4<UNI>(g.aux0, j);
+            const float4 fr = ld4<UNI>(g.aux1, i);
             v2 vi, vj;
             vi.x = fi.x;
             vi.y = fi.y;
@@ -586,18 +608,18 @@ __device__ inline bool intersect_prim(const GeomDev& g, uint32_t prim, v3 o, v3 
             vj.y = fj.y;
             // point_line_segment_distance, fresnel/common/GeometryMath.h:28-39
             const v2 ab = vj - vi;
-            const float Lab = dot(ab, ab);
-            const float s = smax(0.0f, smin(1.0f, dot(p2 - vi, ab) / Lab));
+            const float s = smax(0.0f, smin(1.0f, div_by(dot(p2 - vi, ab), edge_rcp(fr.x, fr.y))));
             const v2 proj = vi + s * ab;
             const v2 dv = p2 - proj;
-            min_d = smin(min_d, sqrtf(dot(dv, dv)));
+            min_sq = smin(min_sq, dot(dv, dv));
             if ((vi.y < p2.y && vj.y >= p2.y) || (vj.y < p2.y && vi.y >= p2.y))
                 {
-                if (vi.x + (p2.y - vi.y) / (vj.y - vi.y) * (vj.x - vi.x) < p2.x)
+                if (vi.x + div_by(p2.y - vi.y, edge_rcp(fr.z, fr.w)) * (vj.x - vi.x) < p2.x)
                     odd = !odd;
                 }
             j = i;
             }
+        const float min_d = smin(3.40282346638528859812e+38f, sqrtf(min_sq));
         float d_edge = odd ? -min_d : min_d;
         if (d_edge > g.rounding)
             return false;

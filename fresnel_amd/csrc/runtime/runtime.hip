@@ -837,8 +837,20 @@ static bool upload_geometry(GeometryObj& g, hipStream_t s)
             }
         else if (g.type == G_POLYGON)
             {
-            for (size_t k = 0; k < g.verts.size() / 2; k++)
-                x0.push_back(make_float4(g.verts[2 * k], g.verts[2 * k + 1], 0.0f, 0.0f));
+            // and, for the edge from vertex k - 1 to k, the reciprocals of its
+            // squared length and of its height as double bits (intersect_prim)
+            const size_t V = g.verts.size() / 2;
+            for (size_t k = 0; k < V; k++)
+                {
+                const float* vi = &g.verts[2 * k];
+                const float* vj = &g.verts[2 * ((k + V - 1) % V)];
+                x0.push_back(make_float4(vi[0], vi[1], 0.0f, 0.0f));
+                const float abx = vj[0] - vi[0], aby = vj[1] - vi[1];
+                const double r[2] = {1.0 / (double)(abx * abx + aby * aby), 1.0 / (double)aby};
+                float4 f;
+                std::memcpy(&f, r, sizeof(f));
+                x1.push_back(f);
+                }
             }
         upload(g.aux0, x0, s);
         upload(g.aux1, x1, s);
@@ -1429,7 +1441,12 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
     // elements: primitives, or (other scenes, tile_group >= 2) the hierarchy
     // cut of kernels/tiles.hip over the N - 1 inner nodes; one more count
     // slot holds the scan's total
-    const bool cut = !spheres && D.tile_group >= 2 && N >= 2;
+    // A polygon's test is the longest (every edge), and a subtree entry runs it
+    // for few lanes at a time, so polygon scenes take subtrees of at most 2
+    // tiles (10,000 hexagons, 641 x 479, 64 samples: primary kernel 2.06 ms at
+    // 4 tiles, 1.79 at 2; meshes 5.16 and 5.11, the mixed scene 7.1 and 7.4).
+    const uint32_t group = scene_types(sc) == (1u << G_POLYGON) ? std::min(D.tile_group, 2u) : D.tile_group;
+    const bool cut = !spheres && group >= 2 && N >= 2;
     const uint32_t n_inner = N - 1;
     const uint32_t n_el = cut ? 2 * n_inner + 2 : N + 1;
     TileTemps& X = D.tile_tmp;
@@ -1443,7 +1460,7 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
                  if (cut)
                      k_tile_cut<false><<<blocks(n_inner + 1, 256), 256, 0, s>>>(
                          sc.nodes.p, n_inner, sc.blo.p, sc.bhi.p, sc.prefix.p, sc.slots.p, sc.n_active, c,
-                         D.tile_group, X.counts.p, X.flags.p, nullptr, nullptr, nullptr, nullptr);
+                         group, X.counts.p, X.flags.p, nullptr, nullptr, nullptr, nullptr);
                  else if (spheres)
                      k_tile_count<true><<<blocks(N + 1, 256), 256, 0, s>>>(sc.blo.p, sc.bhi.p, sc.dgeoms.p, N, c,
                                                                            X.counts.p, X.flags.p);
@@ -1471,7 +1488,7 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
                      if (cut)
                          k_tile_cut<true><<<blocks(n_inner + 1, 256), 256, 0, s>>>(
                              sc.nodes.p, n_inner, sc.blo.p, sc.bhi.p, sc.prefix.p, sc.slots.p, sc.n_active, c,
-                             D.tile_group, X.counts.p, X.flags.p, X.tile0.p, X.q0.p, X.ref0.p, X.valsA.p);
+                             group, X.counts.p, X.flags.p, X.tile0.p, X.q0.p, X.ref0.p, X.valsA.p);
                      else if (spheres)
                          k_tile_emit<true><<<blocks(N, 256), 256, 0, s>>>(sc.blo.p, sc.bhi.p, sc.dgeoms.p, N, c,
                                                                           X.counts.p, X.tile0.p, X.q0.p, X.ref0.p,
