@@ -1043,6 +1043,21 @@ __device__ __forceinline__ uint32_t raster_ordinal(const JobDev& J, uint32_t pix
     return pixel_ordinal(J, pixel - py * J.W, py);
     }
 
+typedef const float __attribute__((address_space(4))) ConstF;
+typedef const uint32_t __attribute__((address_space(4))) ConstU;
+
+// Whether chunk c (64 pixels of the primary order, the same for the whole
+// wavefront) is a full tile whose candidate list is empty: every ray of its
+// pixels misses.  Nothing is traced, shaded or recorded for such a chunk;
+// k_accumulate and k_preview take its samples as background.
+__device__ __forceinline__ bool empty_chunk(const JobDev& J, uint32_t c)
+    {
+    if (!J.use_tiles || c >= J.tiles_x * J.tiles_y)
+        return false;
+    c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
+    return ((const ConstU*)J.tile_start)[c] == ((const ConstU*)J.tile_end)[c];
+    }
+
 __device__ __forceinline__ void primary_order(const JobDev& J, uint32_t local, uint32_t& k, uint32_t& px,
                                               uint32_t& py, uint32_t& j)
     {
@@ -1510,8 +1525,6 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(LOOP ? 7 : 1
 // majority, and pushes the other with each lane's own cull bound.  A group of
 // 64 rays that straddles jobs is searched once for each.
 constexpr uint32_t UNWANTED = 0x80000000u; // stack flag: this lane does not need the node
-typedef const float __attribute__((address_space(4))) ConstF;
-typedef const uint32_t __attribute__((address_space(4))) ConstU;
 typedef const GeomDev __attribute__((address_space(4))) ConstGeom;
 
 // Leaf test of a primitive every lane of the wavefront shares: the geometry
@@ -1947,10 +1960,33 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == 
             {
             const JobDev& J = jobs[job];
             const uint32_t end = (job == job_last) ? n : jobs[job + 1].ray_base;
+            // chunks of 64 pixels of this job's first and last ray here
+            const uint32_t c0 = fdiv(max(base, J.ray_base) - J.ray_base, J.div_chunk);
+            const uint32_t c1 = fdiv(min(last + 1u, end) - 1u - J.ray_base, J.div_chunk);
+            if (c0 == c1 && empty_chunk(J, c0))
+                {
+                if (COUNT)
+                    for (uint32_t g = 0; g < groups; g++)
+                        {
+                        const uint32_t i = base + (wave * groups + g) * 64 + lane;
+                        n_rays += (i >= J.ray_base && i < end) ? 1u : 0u;
+                        }
+                continue;
+                }
             for (uint32_t g = 0; g < groups; g++)
                 {
-                const uint32_t i = base + (wave * groups + g) * 64 + lane;
-                const bool valid = i >= J.ray_base && i < end;
+                const uint32_t i0 = base + ((uint32_t)__builtin_amdgcn_readfirstlane((int)wave) * groups + g) * 64;
+                const uint32_t i = i0 + lane;
+                bool valid = i >= J.ray_base && i < end;
+                if (COUNT && valid)
+                    n_rays++;
+                if (c0 != c1 && i0 >= J.ray_base && i0 < end)
+                    {
+                    // the group's chunk, if its rays belong to one
+                    const uint32_t a = fdiv(i0 - J.ray_base, J.div_chunk);
+                    if (a == fdiv(min(i0 + 64u, end) - 1u - J.ray_base, J.div_chunk) && empty_chunk(J, a))
+                        valid = false;
+                    }
                 v3 o = mk3(0.0f, 0.0f, 0.0f), d = mk3(0.0f, 0.0f, 1.0f);
                 uint32_t k = 0, px = 0, py = 0, jord = 0;
                 if (valid)
@@ -1961,8 +1997,6 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == 
                 best.prim = EMPTY;
                 primary_group_hit<SS, COUNT, TYPES, true>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes,
                                                           n_prims, n_entries, err);
-                if (COUNT && valid)
-                    n_rays++;
                 shade_primary_block<BLOCK, TYPES>(jobs, valid, job, k, py * J.W + px, jord, o, d, best, out, seg,
                                                   records, sh);
                 }
@@ -2320,6 +2354,10 @@ __global__ void k_accumulate(const JobDev* __restrict__ jobs, const uint32_t* __
     const uint32_t pixel = py * J.W + px;
     float4 mean = J.linear[pixel];
     const uint32_t K = J.K;
+    // a chunk nothing was traced for has no records (empty_chunk; a wavefront
+    // of a later job may straddle two chunks)
+    const uint32_t chunk = jord >> 6;
+    const bool empty = J.use_tiles && chunk < J.tiles_x * J.tiles_y && J.tile_start[chunk] == J.tile_end[chunk];
     // the first records of four camera samples are loaded together, then
     // folded into the mean in sample order
     constexpr uint32_t U = 4;
@@ -2328,7 +2366,7 @@ __global__ void k_accumulate(const JobDev* __restrict__ jobs, const uint32_t* __
     uint4 rk[U];
 #pragma unroll
     for (uint32_t u = 0; u < U; u++)
-        rk[u] = (k0 + u < K) ? records[rec_index(J, k0 + u, jord, 0)] : make_uint4(0, 0, 0, 0);
+        rk[u] = (k0 + u < K && !empty) ? records[rec_index(J, k0 + u, jord, 0)] : make_uint4(0, 0, 0, REC_BG);
 #pragma unroll
     for (uint32_t u = 0; u < U; u++)
         {
@@ -2478,7 +2516,22 @@ __global__ __launch_bounds__(BLOCK) void k_preview(const JobDev* __restrict__ jo
         if (valid)
             ordinal_pixel(J, j, px, py);
         float4 sum = make_float4(0, 0, 0, 0); // SPLIT: .x is this thread's channel
-        const uint32_t rounds = SPLIT ? (samples + WAVES - 1) / WAVES : samples;
+        uint32_t rounds = SPLIT ? (samples + WAVES - 1) / WAVES : samples;
+        if (empty_chunk(J, SPLIT ? chunk : (uint32_t)__builtin_amdgcn_readfirstlane((int)chunk)))
+            {
+            // every sample is background, added as often
+            const uint32_t ch = threadIdx.x & 3u;
+            const float4 b = make_float4(J.bg.x, J.bg.y, J.bg.z, J.bg_alpha);
+            const float x = (ch == 0u) ? b.x : (ch == 1u) ? b.y : (ch == 2u) ? b.z : b.w;
+            for (uint32_t k = 0; k < samples; k++)
+                {
+                sum.x += SPLIT ? x : b.x;
+                sum.y += b.y;
+                sum.z += b.z;
+                sum.w += b.w;
+                }
+            rounds = 0;
+            }
         for (uint32_t r = 0; r < rounds; r++)
             {
             const uint32_t sample = SPLIT ? r * WAVES + wave : r;
