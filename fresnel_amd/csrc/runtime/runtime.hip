@@ -1653,7 +1653,7 @@ struct BatchExec
     bool spheres;
     std::vector<uint32_t> pix_base;
     uint64_t n_pri = 0, n_paths = 0, n_pix = 0, n_rec = 0;
-    uint32_t nj = 0, gstride = 0, seg_cap = 0, tail_threads = 0, rest_grid = 0;
+    uint32_t nj = 0, gstride = 0, seg_cap = 0, tail_threads = 0, rest_grid = 0, tail_grid = 0;
     uint32_t pgroups = 1; // primary claim size in workgroups of rays (primary_groups)
     uint32_t n_steps = 0;
     int cur = 1;
@@ -1767,6 +1767,17 @@ struct BatchExec
         rest_grid = D.grid_for(reinterpret_cast<const void*>(spheres ? k_shade<SHADE_BLOCK, T_SPHERES, true>
                                                                      : k_shade<SHADE_BLOCK, T_ALL, true>),
                                SHADE_BLOCK);
+        // resident grid of the tail kernel, within its overflow stacks
+        tail_grid = std::min(D.grid_for(reinterpret_cast<const void*>(finish_kernel()), TRAV_BLOCK),
+                             tail_threads / TRAV_BLOCK);
+        }
+
+    auto finish_kernel() const -> decltype(&k_finish<TRAV_BLOCK, TRAV_SS, false, T_ALL>)
+        {
+        return spheres ? (D.count_on ? k_finish<TRAV_BLOCK, TRAV_SS, true, T_SPHERES>
+                                     : k_finish<TRAV_BLOCK, TRAV_SS, false, T_SPHERES>)
+                       : (D.count_on ? k_finish<TRAV_BLOCK, TRAV_SS, true, T_ALL>
+                                     : k_finish<TRAV_BLOCK, TRAV_SS, false, T_ALL>);
         }
 
     // Workgroups of the one-unit shading launch at bounce step b: the live
@@ -1791,7 +1802,7 @@ struct BatchExec
         std::vector<uint64_t> k = {(uint64_t)(uintptr_t)s, nj, n_pri, n_paths, n_pix, n_rec, seg_cap, gstride,
                                    tail_threads, types, steps, D.trav_chunk, pgroups, D.xcd_bands,
                                    D.fuse_primary, D.fuse_bounce, D.tail_rays, (uint64_t)D.stack_lds, D.trav_refill,
-                                   D.trav_packet, D.count_on ? 1u : 0u, rest_grid};
+                                   D.trav_packet, D.count_on ? 1u : 0u, rest_grid, tail_grid};
         for (const void* p : {(const void*)R.qo[0].p, (const void*)R.qo[1].p, (const void*)R.qd[0].p,
                               (const void*)R.qd[1].p, (const void*)R.qatt[0].p, (const void*)R.qatt[1].p,
                               (const void*)R.qmeta[0].p, (const void*)R.qmeta[1].p, (const void*)R.hits.p,
@@ -1838,6 +1849,7 @@ struct BatchExec
     // finishes every path that is still queued.
     void enqueue_steps(uint32_t steps)
         {
+        auto* f = finish_kernel();
         auto* shade_one = spheres ? k_shade<SHADE_BLOCK, T_SPHERES, false> : k_shade<SHADE_BLOCK, T_ALL, false>;
         auto* shade_rest = spheres ? k_shade<SHADE_BLOCK, T_SPHERES, true> : k_shade<SHADE_BLOCK, T_ALL, true>;
         for (uint32_t b = 0; b < steps; b++)
@@ -1888,13 +1900,9 @@ struct BatchExec
             launch("finish",
                    [&]
                    {
-                       auto* f = spheres ? (D.count_on ? k_finish<TRAV_BLOCK, TRAV_SS, true, T_SPHERES>
-                                                       : k_finish<TRAV_BLOCK, TRAV_SS, false, T_SPHERES>)
-                                         : (D.count_on ? k_finish<TRAV_BLOCK, TRAV_SS, true, T_ALL>
-                                                       : k_finish<TRAV_BLOCK, TRAV_SS, false, T_ALL>);
-                       f<<<tail_threads / TRAV_BLOCK, TRAV_BLOCK, 0, s>>>(R.jobs.p, nj, in, 0u, R.view.p,
-                                                                          R.records.p, MAX_DEPTH, R.tail_stack.p,
-                                                                          tail_threads, D.counters.p);
+                       f<<<tail_grid, TRAV_BLOCK, 0, s>>>(R.jobs.p, nj, in, 0u, R.view.p, R.counters32.p,
+                                                          R.records.p, MAX_DEPTH, R.tail_stack.p,
+                                                          tail_grid * TRAV_BLOCK, D.counters.p);
                    });
             D.tag_mode = nullptr;
             cur = 1 - cur;
