@@ -15,7 +15,7 @@ for every setting; only speed changes.  Knobs (see fh_device_tune):
 * ``primary_chunk`` the most primary rays a workgroup claims at once (a
                   batch with fewer than 16 such claims per CU claims less).
 * ``trav_refill`` idle lanes of a traversal wavefront that trigger taking new
-                  rays (65: trace 64 rays at a time).
+                  rays (64 or 65: all of them).
 * ``trav_packet`` primary rays traced as wavefront packets (2) or per ray (1).
 * ``primary_tiles`` primary rays tested against per-tile candidate lists (2)
                   or searched in the BVH (1).  With lists on, a tracer builds

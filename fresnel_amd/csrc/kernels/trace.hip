@@ -419,11 +419,13 @@ __device__ inline void trace_binary(const SceneDev& sc, v3 o, v3 d, float tnear,
 // are tested later, many lanes together:
 //   * a child box is 8-bit steps of the node's interval (k_bvh4_fill); the
 //     ray's direction signs pick the near and far ends, so an axis of a
-//     child's slab interval is two byte conversions and two fmas.  The node's
-//     pad and the ray's (2^-20 of the largest coordinate of node and origin
-//     each, against rounding errors of at most 7 and 6 x 2^-24 of them) make
-//     the interval contain, on every axis, the float slab interval
-//     (lo - o) * inv of every primitive inside;
+//     child's slab interval is two byte conversions and two fmas.  The
+//     rounding of these (the node's origin less the ray's, exact operands, is
+//     one rounding) and of a primitive's float slab interval (lo - o) * inv
+//     is at most 5 x 2^-24 of the interval's end and 6 x 2^-24 of the node's
+//     largest coordinate times the reciprocal; the node's pad (2^-20 of that
+//     coordinate) and the factor 1 + 2^-19 in the comparison cover them, so
+//     every child whose primitives' own test could pass is open;
 //   * the exact slab gate of a primitive's own bounds and its intersector run
 //     at the leaf step.  Leaf children are sorted and pushed like inner ones;
 //     a lane that takes one waits until enough lanes hold one.
@@ -470,8 +472,7 @@ template<> struct SearchScene<false>
 
 struct Search
     {
-    v3 o, d, inv;     // the ray; exact reciprocals for the primitives' gates
-    v3 ic, near, far; // node tests: bounded reciprocals, -o * ic less and plus the pad
+    v3 o, d, ic;      // the ray; reciprocals of d, bounded (node_rcp)
     float tnear;
     float margin;
     float cull;       // best.t + margin
@@ -480,12 +481,26 @@ struct Search
     };
 
 // Reciprocal of a direction component for the node tests.  Below 2^-60 it is
-// taken as 2^60: a box the origin lies beside by more than the pads is missed,
-// and inside one the interval reaches 2^40 times the largest coordinate, past
-// every hit.
-__device__ __forceinline__ float node_rcp(float d, float inv)
+// taken as 2^60: a box the origin lies beside by more than the node's pad is
+// missed, and inside one the interval reaches 2^40 times the node's largest
+// coordinate, past every hit.
+constexpr float RCP_MAX = 0x1p60f;
+__device__ __forceinline__ float node_rcp(float d)
     {
-    return (fabsf(d) < 0x1p-60f) ? copysignf(0x1p60f, d) : inv;
+    const float inv = 1.0f / d;
+    return (fabsf(d) < 1.0f / RCP_MAX) ? copysignf(RCP_MAX, d) : inv;
+    }
+// The exact reciprocals, for the gate of a primitive's own bounds.
+__device__ __forceinline__ v3 exact_rcp(const Search& r)
+    {
+    v3 i = r.ic;
+    if (fabsf(i.x) == RCP_MAX)
+        i.x = 1.0f / r.d.x;
+    if (fabsf(i.y) == RCP_MAX)
+        i.y = 1.0f / r.d.y;
+    if (fabsf(i.z) == RCP_MAX)
+        i.z = 1.0f / r.d.z;
+    return i;
     }
 
 template<class Stack>
@@ -493,13 +508,7 @@ __device__ __forceinline__ void search_begin(const SceneDev& sc, v3 o, v3 d, flo
     {
     r.o = o;
     r.d = d;
-    r.inv = mk3(1.0f / d.x, 1.0f / d.y, 1.0f / d.z);
-    r.ic = mk3(node_rcp(d.x, r.inv.x), node_rcp(d.y, r.inv.y), node_rcp(d.z, r.inv.z));
-    const v3 n = mk3(-(o.x * r.ic.x), -(o.y * r.ic.y), -(o.z * r.ic.z));
-    const float om = fmaxf(fmaxf(fabsf(o.x), fabsf(o.y)), fabsf(o.z)) * NODE_PAD;
-    const v3 pad = mk3(om * fabsf(r.ic.x), om * fabsf(r.ic.y), om * fabsf(r.ic.z));
-    r.near = n - pad;
-    r.far = n + pad;
+    r.ic = mk3(node_rcp(d.x), node_rcp(d.y), node_rcp(d.z));
     r.tnear = tnear;
     r.margin = sc.cull_margin;
     r.cull = __builtin_huge_valf();
@@ -552,9 +561,7 @@ __device__ __forceinline__ void search_visit(const Node4* __restrict__ nodes, Se
     const float ox = __uint_as_float(A.x), oy = __uint_as_float(A.y), oz = __uint_as_float(A.z);
     const float sx = __uint_as_float(A.w) * r.ic.x, sy = __uint_as_float(B.x) * r.ic.y,
                 sz = __uint_as_float(B.y) * r.ic.z;
-    const float nx = __builtin_fmaf(ox, r.ic.x, r.near.x), fx = __builtin_fmaf(ox, r.ic.x, r.far.x);
-    const float ny = __builtin_fmaf(oy, r.ic.y, r.near.y), fy = __builtin_fmaf(oy, r.ic.y, r.far.y);
-    const float nz = __builtin_fmaf(oz, r.ic.z, r.near.z), fz = __builtin_fmaf(oz, r.ic.z, r.far.z);
+    const float bx = (ox - r.o.x) * r.ic.x, by = (oy - r.o.y) * r.ic.y, bz = (oz - r.o.z) * r.ic.z;
     const bool px = r.ic.x >= 0.0f, py = r.ic.y >= 0.0f, pz = r.ic.z >= 0.0f;
     const uint32_t qnx = px ? B.z : C.y, qfx = px ? C.y : B.z;
     const uint32_t qny = py ? B.w : C.z, qfy = py ? C.z : B.w;
@@ -565,11 +572,11 @@ __device__ __forceinline__ void search_visit(const Node4* __restrict__ nodes, Se
     for (int k = 0; k < 4; k++)
         {
         auto byte = [k](uint32_t q) { return (float)((q >> (8 * k)) & 0xffu); };
-        const float tx = __builtin_fmaf(byte(qnx), sx, nx), ux = __builtin_fmaf(byte(qfx), sx, fx);
-        const float ty = __builtin_fmaf(byte(qny), sy, ny), uy = __builtin_fmaf(byte(qfy), sy, fy);
-        const float tz = __builtin_fmaf(byte(qnz), sz, nz), uz = __builtin_fmaf(byte(qfz), sz, fz);
+        const float tx = __builtin_fmaf(byte(qnx), sx, bx), ux = __builtin_fmaf(byte(qfx), sx, bx);
+        const float ty = __builtin_fmaf(byte(qny), sy, by), uy = __builtin_fmaf(byte(qfy), sy, by);
+        const float tz = __builtin_fmaf(byte(qnz), sz, bz), uz = __builtin_fmaf(byte(qfz), sz, bz);
         const float lo = fmaxf(fmaxf(fmaxf(tx, ty), tz), 0.0f);
-        const float hi = fminf(fminf(ux, uy), uz);
+        const float hi = fminf(fminf(ux, uy), uz) * (1.0f + 0x1p-19f);
         const float q = __builtin_fmaf(-CULL_K, hi, lo);
         const bool open = (lo <= hi) & !(q > r.cull) & (k < 2 || nd[k] != EMPTY);
         key[k] = open ? q : __builtin_huge_valf();
@@ -597,7 +604,7 @@ __device__ __forceinline__ void search_sphere(const SearchScene<UNI>& sc, Search
     const uint32_t p = r.cur & ~LEAF;
     const float4 s = ldg(sc.leaf(), p);
     float tmin, tmax;
-    slab(r.o, r.inv, s.x - s.w, s.y - s.w, s.z - s.w, s.x + s.w, s.y + s.w, s.z + s.w, tmin, tmax);
+    slab(r.o, exact_rcp(r), s.x - s.w, s.y - s.w, s.z - s.w, s.x + s.w, s.y + s.w, s.z + s.w, tmin, tmax);
     if (!((tmin <= tmax) && (tmax >= r.tnear)))
         return;
     if (COUNT)
@@ -656,7 +663,7 @@ __device__ __forceinline__ void search_mixed(const SearchScene<UNI>& sc, Search&
     const uint32_t p = r.cur & ~LEAF;
     const float4 a = ldg(sc.leaf(), 2 * (size_t)p), b = ldg(sc.leaf(), 2 * (size_t)p + 1);
     float tmin, tmax;
-    slab(r.o, r.inv, a.x, a.y, a.z, b.x, b.y, b.z, tmin, tmax);
+    slab(r.o, exact_rcp(r), a.x, a.y, a.z, b.x, b.y, b.z, tmin, tmax);
     if (!((tmin <= tmax) && (tmax >= r.tnear)))
         return;
     const uint32_t slot = __float_as_uint(a.w), prim = __float_as_uint(b.w);
@@ -1148,20 +1155,26 @@ struct Claims
         }
     };
 
-// Held to 72 registers (7 wavefronts per SIMD): at 6, 7, 8 the lattice of 1M
-// spheres takes 9.3, 9.2, 10.2 ms of traversal; at 5, 6, 7, 8 the mixed scene
-// takes 10.7, 10.0, 9.5, 10.9 ms and the mesh scene 9.7, 9.2, 9.2, 10.4 ms
-// (fewer wavefronts hide less of the node loads, at 8 values of the search
-// spill).  Before the 4-wide search of all scene types those scenes took
-// 11.4, 14.4 and 15.3 ms.
+// Each wavefront searches 64 rays at a time and takes new ones as soon as
+// `refill` lanes are idle, so lanes do not wait for the longest ray of 64.  A
+// wavefront's rays belong to one job at a time (nearly all chunks do: the
+// queues are filled chunk by chunk), whose scene pointers are scalar.  Bound
+// by VALU issue and the latency of node and leaf loads.  Traversal per call
+// with 64 rays at a time to their ends, and so: lattice of 1M spheres 9.0 and
+// 8.3 ms, small scene 0.55 and 0.36, meshes 9.1 and 6.0, mixed 9.5 and 5.9,
+// spherocylinders 2.2 and 1.0 (refill at 16, 24, 32, 40 idle lanes: lattice
+// 8.8, 8.7, 8.4, 8.1, meshes 6.1, 6.0, 6.2, 6.3, mixed 5.95, 5.98, 6.01, 6.19).
+// Held to 7 wavefronts per SIMD in spheres-only scenes (6: lattice 8.8; 8
+// spills), 6 otherwise (5: mixed 6.4, 7: meshes 7.5 against 6.9 then).
 template<int BLOCK, int SS, bool COUNT, bool PRIMARY, uint32_t TYPES>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void k_traverse(
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == T_SPHERES ? 7 : 6))) void k_traverse(
     const JobDev* __restrict__ jobs, uint32_t n_jobs, Queue q, uint32_t n, const QueueView* __restrict__ view,
-    uint4* hits, uint32_t* work, uint32_t chunk, uint32_t bands, uint2* gstack, uint32_t gstride,
+    uint4* hits, uint32_t* work, uint32_t chunk, uint32_t bands, uint32_t refill, uint2* gstack, uint32_t gstride,
     unsigned long long* counters)
     {
     if (!take_view(view, VIEW_BOUNCE, q, n))
         return;
+    constexpr uint32_t LEAF_WAIT = TYPES == T_SPHERES ? 1 : 2;
     __shared__ uint2 lds[SS * BLOCK];
     const uint32_t gtid = blockIdx.x * BLOCK + threadIdx.x;
     LdsStack<SS> st;
@@ -1171,66 +1184,129 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7))) void
     st.gstride = gstride;
     st.sp = 0;
     const uint32_t lane = lane_id();
+    const uint64_t below = (1ull << lane) - 1ull;
     uint32_t n_nodes = 0, n_prims = 0, err = 0, n_rays = 0;
     Claims cl;
     cl.work = work;
-    cl.chunk = chunk;
+    // at least eight claims a wavefront, down to 64 rays each: a launch of a few
+    // million rays in claims of 256 leaves half the wavefronts without work
+    // (claims of 256: small scene 0.48 ms, meshes 7.0, mixed 6.5; two, four,
+    // eight, sixteen claims a wavefront: mixed 6.05, 6.01, 5.86, 5.75, lattice
+    // 8.35, 8.40, 8.35, 8.42)
+    const uint32_t share = n / (gridDim.x * (BLOCK / 64) * 8);
+    cl.chunk = max(64u, min(chunk, share & ~63u));
     cl.n = n;
     cl.ranges = (bands && !PRIMARY) ? 8u : 1u;
     cl.r = (cl.ranges == 8u) ? (blockIdx.x & 7u) : 0u;
     cl.tried = 0;
-    uint32_t base, end;
-    cl.next(q, lane, base, end);
-    while (base != EMPTY)
+    uint32_t pool, pool_end; // untaken rays of the wavefront's chunk; the next chunk is claimed ahead
+    uint32_t next, next_end;
+    cl.next(q, lane, pool, pool_end);
+    cl.next(q, lane, next, next_end);
+    uint32_t job = 0; // of every ray the wavefront holds
+    Search r;
+    r.cur = EMPTY;
+    uint32_t i = EMPTY; // the lane's ray (EMPTY: none)
+    for (;;)
         {
-        uint32_t nbase, nend; // the next chunk, claimed before tracing this one
-        cl.next(q, lane, nbase, nend);
-        for (uint32_t sub = base; sub < end; sub += 64)
-        {
-        const uint32_t i = sub + lane;
-        const uint32_t sl = PRIMARY ? 0u : q_slot(q, i, sub, min(end, sub + 64u) - 1u);
-        if (i < end)
+        // store finished rays, take new ones
+        const uint32_t n_idle = (uint32_t)__popcll(__ballot(r.cur == EMPTY));
+        const bool stop = n_idle >= refill || n_idle == 64;
+        const SearchScene<true> done(jobs[job].scene);
+        if (stop && r.cur == EMPTY && i != EMPTY)
             {
-            v3 o, d;
-            float tnear;
-            uint32_t job;
-            if (PRIMARY)
-                {
-                uint32_t k, pixel, jord;
-                primary_ray(jobs, n_jobs, i, job, k, pixel, jord, o, d);
-                tnear = 1e-3f;
-                }
-            else
-                {
-                const float4 a = q.o[sl];
-                const float4 b = q.d[sl];
-                o = mk3(a.x, a.y, a.z);
-                d = mk3(b.x, b.y, b.z);
-                tnear = a.w;
-                job = __float_as_uint(b.w);
-                }
-            // one job at a time, so that the scene's pointers are scalar: nearly
-            // every wavefront's rays belong to one (the queues are filled chunk by
-            // chunk, a chunk's rays by one job)
-            HitT h;
-            for (bool todo = true; __ballot(todo) != 0;)
-                if (todo)
-                    {
-                    const uint32_t j0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)job);
-                    if (job == j0)
-                        {
-                        trace_closest<LdsStack<SS>, COUNT, TYPES, true>(jobs[j0].scene, o, d, tnear, h, st, n_nodes,
-                                                                        n_prims, err);
-                        todo = false;
-                        }
-                    }
+            const HitT h = search_end<TYPES, true>(done, r);
             hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, 0);
+            i = EMPTY;
             if (COUNT)
                 n_rays++;
             }
-        }
-        base = nbase;
-        end = nend;
+        bool blocked = false; // the next unclaimed ray belongs to another job
+        while (stop && pool != EMPTY && !blocked)
+            {
+            const uint64_t need = __ballot(i == EMPTY);
+            if (need == 0)
+                break;
+            const uint32_t avail = pool_end - pool;
+            const uint32_t rank = (uint32_t)__popcll(need & below);
+            const bool take = i == EMPTY && rank < avail;
+            uint32_t took = min((uint32_t)__popcll(need), avail);
+            v3 o = mk3(0, 0, 0), d = mk3(0, 0, 1);
+            float tnear = 1e-3f;
+            uint32_t j = 0;
+            if (take)
+                {
+                if (PRIMARY)
+                    {
+                    uint32_t k, pixel, jord;
+                    primary_ray(jobs, n_jobs, pool + rank, j, k, pixel, jord, o, d);
+                    }
+                else
+                    {
+                    const uint32_t sl = q_slot(q, pool + rank, pool, pool_end - 1u);
+                    const float4 a = q.o[sl];
+                    const float4 b = q.d[sl];
+                    o = mk3(a.x, a.y, a.z);
+                    d = mk3(b.x, b.y, b.z);
+                    tnear = a.w;
+                    j = __float_as_uint(b.w);
+                    }
+                }
+            bool mine = take;
+            if (n_jobs > 1)
+                {
+                // rays of one job at a time: an idle wavefront takes its first
+                // ray's job, the rays before the first of another job are taken
+                const uint32_t first = (uint32_t)(__ffsll((unsigned long long)need) - 1);
+                if (need == ~0ull)
+                    job = (uint32_t)__builtin_amdgcn_readlane((int)j, first);
+                const uint64_t other = __ballot(take && j != job);
+                if (other != 0)
+                    {
+                    blocked = true;
+                    took = (uint32_t)__popcll(need & ((other & (~other + 1ull)) - 1ull));
+                    mine = take && rank < took;
+                    }
+                }
+            if (mine)
+                {
+                i = pool + rank;
+                search_begin(jobs[job].scene, o, d, tnear, r, st);
+                }
+            pool += took;
+            if (pool == pool_end)
+                {
+                pool = next;
+                pool_end = next_end;
+                if (next != EMPTY)
+                    cl.next(q, lane, next, next_end);
+                }
+            }
+        if (__ballot(r.cur != EMPTY) == 0)
+            {
+            if (__ballot(i != EMPTY) == 0)
+                break;
+            continue; // rays of an empty scene: stored above
+            }
+        const SearchScene<true> sc(jobs[job].scene);
+        const bool more = pool != EMPTY && !blocked;
+        uint32_t n_in, n_leaf;
+        for (;;)
+            {
+            const bool inner = !(r.cur & LEAF);
+            n_in = (uint32_t)__popcll(__ballot(inner));
+            n_leaf = (uint32_t)__popcll(__ballot((r.cur & LEAF) && r.cur != EMPTY));
+            if (n_in == 0 || n_leaf >= LEAF_WAIT * n_in || (more && n_in + n_leaf + refill <= 64))
+                break;
+            if (inner)
+                search_visit<LdsStack<SS>, COUNT>(sc.nodes4(), r, st, n_nodes, err);
+            }
+        if (n_leaf != 0 && n_leaf >= LEAF_WAIT * n_in)
+            if ((r.cur & LEAF) && r.cur != EMPTY)
+                {
+                search_leaf<TYPES, COUNT, true>(sc, r, n_prims);
+                search_pop(r, st);
+                }
         }
     if (COUNT)
         {
@@ -2102,147 +2178,6 @@ __global__ __launch_bounds__(BLOCK) void k_bounce(const JobDev* __restrict__ job
         atomicAdd(counters + CTR_SECONDARY + 0, (unsigned long long)n_rays);
         atomicAdd(counters + CTR_SECONDARY + 1, (unsigned long long)n_nodes);
         atomicAdd(counters + CTR_SECONDARY + 2, (unsigned long long)n_prims);
-        }
-    if (err)
-        atomicOr((unsigned int*)(counters + CTR_OVERFLOW), 1u);
-    }
-
-// Persistent traversal with per-lane refill: a lane whose ray is finished
-// starts a new one as soon as at least `refill` lanes of the wavefront are
-// idle (or all are), so lanes do not wait for the slowest ray of a 64-ray
-// batch.  Every lane holds its next ray already loaded: a refill starts the
-// prefetched ray from registers and issues the loads of the one after it,
-// which arrive while the wavefront keeps searching, so a refill never waits
-// on memory.  Rays are claimed per wavefront from the chunks of Claims (XCD
-// bands as in k_traverse).  Same per-ray arithmetic as k_traverse.
-template<int BLOCK, int SS, bool COUNT, bool PRIMARY, uint32_t TYPES>
-__global__ __launch_bounds__(BLOCK) void k_traverse_dyn(const JobDev* __restrict__ jobs, uint32_t n_jobs, Queue q,
-                                                        uint32_t n, const QueueView* __restrict__ view, uint4* hits,
-                                                        uint32_t* work, uint32_t chunk, uint32_t bands,
-                                                        uint32_t refill, uint2* gstack, uint32_t gstride,
-                                                        unsigned long long* counters)
-    {
-    if (!take_view(view, VIEW_BOUNCE, q, n))
-        return;
-    __shared__ uint2 lds[SS * BLOCK];
-    const uint32_t gtid = blockIdx.x * BLOCK + threadIdx.x;
-    LdsStack<SS> st;
-    st.lds = lds + threadIdx.x;
-    st.lstride = BLOCK;
-    st.glob = gstack + gtid;
-    st.gstride = gstride;
-    st.sp = 0;
-    const uint32_t lane = lane_id();
-    const uint64_t below = (1ull << lane) - 1ull;
-    uint32_t n_nodes = 0, n_prims = 0, err = 0, n_rays = 0;
-    Claims cl;
-    cl.work = work;
-    cl.chunk = chunk;
-    cl.n = n;
-    cl.ranges = (bands && !PRIMARY) ? 8u : 1u;
-    cl.r = (cl.ranges == 8u) ? (blockIdx.x & 7u) : 0u;
-    cl.tried = 0;
-    uint32_t pool, pool_end;
-    cl.next(q, lane, pool, pool_end);
-    // the lane's prefetched ray: index, origin + tnear, direction + job
-    uint32_t pf = EMPTY;
-    float4 pa = make_float4(0, 0, 0, 0), pb = make_float4(0, 0, 1, 0);
-    // Give every lane without a prefetched ray the next unclaimed ray, in
-    // lane order, and issue its loads (not waited for here).
-    auto prefetch = [&]()
-    {
-        for (;;)
-            {
-            const uint64_t need = __ballot(pf == EMPTY);
-            if (need == 0 || pool == EMPTY)
-                return;
-            const uint32_t avail = pool_end - pool;
-            const uint32_t rank = (uint32_t)__popcll(need & below);
-            if (pf == EMPTY && rank < avail)
-                {
-                pf = pool + rank;
-                if (PRIMARY)
-                    {
-                    pa = make_float4(0, 0, 0, 1e-3f);
-                    pb = make_float4(0, 0, 1, 0);
-                    }
-                else
-                    {
-                    const uint32_t sl = q_slot(q, pf, pool, pool_end - 1u);
-                    pa = q.o[sl];
-                    pb = q.d[sl];
-                    }
-                }
-            const uint32_t took = min((uint32_t)__popcll(need), avail);
-            pool += took;
-            if (pool < pool_end)
-                return;
-            cl.next(q, lane, pool, pool_end);
-            }
-    };
-    prefetch();
-    bool active = false;
-    uint32_t i = 0;
-    Search r;
-    uint32_t job = 0;
-    for (;;)
-        {
-        const uint32_t n_idle = (uint32_t)__popcll(__ballot(!active));
-        const uint64_t ready = __ballot(!active && pf != EMPTY);
-        if (ready != 0 && (n_idle >= refill || n_idle == 64))
-            {
-            if (!active && pf != EMPTY)
-                {
-                i = pf;
-                pf = EMPTY;
-                v3 o, d;
-                float tnear;
-                if (PRIMARY)
-                    {
-                    uint32_t k, pixel, jord;
-                    primary_ray(jobs, n_jobs, i, job, k, pixel, jord, o, d);
-                    tnear = 1e-3f;
-                    }
-                else
-                    {
-                    o = mk3(pa.x, pa.y, pa.z);
-                    d = mk3(pb.x, pb.y, pb.z);
-                    tnear = pa.w;
-                    job = __float_as_uint(pb.w);
-                    }
-                search_begin(jobs[job].scene, o, d, tnear, r, st);
-                active = true;
-                }
-            prefetch();
-            }
-        if (__ballot(active) == 0)
-            break;
-        if (active)
-            {
-            const SearchScene<false> sc(jobs[job].scene);
-            if (!(r.cur & LEAF))
-                search_visit<LdsStack<SS>, COUNT>(sc.nodes4(), r, st, n_nodes, err);
-            else if (r.cur != EMPTY)
-                {
-                search_leaf<TYPES, COUNT, false>(sc, r, n_prims);
-                search_pop(r, st);
-                }
-            }
-        if (active && r.cur == EMPTY)
-            {
-            const HitT h = search_end<TYPES, false>(jobs[job].scene, r);
-            hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, 0);
-            active = false;
-            if (COUNT)
-                n_rays++;
-            }
-        }
-    if (COUNT)
-        {
-        const int c = PRIMARY ? CTR_PRIMARY : CTR_SECONDARY;
-        atomicAdd(counters + c + 0, (unsigned long long)n_rays);
-        atomicAdd(counters + c + 1, (unsigned long long)n_nodes);
-        atomicAdd(counters + c + 2, (unsigned long long)n_prims);
         }
     if (err)
         atomicOr((unsigned int*)(counters + CTR_OVERFLOW), 1u);

@@ -278,8 +278,8 @@ struct DeviceObj
     uint32_t fuse_bounce = 1;           // 2: secondary traversal and shading in one kernel, 1: two
     uint32_t inflight = 2;              // batches of one Path.sample in flight (1 or 2)
     uint32_t xcd_bands = 2;             // 2: queue segments hold image bands, traversal claims per XCD; 1: off
-    uint32_t trav_refill = 65;          // lanes take new rays once this many of a wavefront are idle
-                                        // (65: batch-synchronous kernel, 64 rays at a time)
+    uint32_t trav_refill = 32;          // lanes take new rays once this many of a wavefront are idle
+                                        // (64 and more: all of them)
     int stack_lds = 8;                  // traversal stack entries kept in LDS (8 or 16)
     std::map<const void*, uint32_t> grids;
     uint32_t grid_for(const void* kernel, int block)
@@ -408,20 +408,6 @@ static void launch_traverse(DeviceObj& D, const char* nm, hipStream_t s, const T
                  });
         return;
         }
-    if (D.trav_refill <= 64)
-        {
-        auto kern = &k_traverse_dyn<TRAV_BLOCK, SS, C, P, T>;
-        const uint32_t grid = D.grid_for(reinterpret_cast<const void*>(kern), TRAV_BLOCK);
-        REQUIRE((uint64_t)grid * TRAV_BLOCK <= a.gstride, "traversal grid exceeds the overflow stacks");
-        D.launch(nm,
-                 [&]
-                 {
-                     kern<<<grid, TRAV_BLOCK, 0, s>>>(a.jobs, a.n_jobs, a.q, a.n, a.view, a.hits, a.work, a.chunk,
-                                                     D.xcd_bands == 2 ? 1u : 0u, D.trav_refill, a.gstack,
-                                                     a.gstride, a.counters);
-                 });
-        return;
-        }
     auto kern = &k_traverse<TRAV_BLOCK, SS, C, P, T>;
     const uint32_t grid = D.grid_for(reinterpret_cast<const void*>(kern), TRAV_BLOCK);
     REQUIRE((uint64_t)grid * TRAV_BLOCK <= a.gstride, "traversal grid exceeds the overflow stacks");
@@ -429,7 +415,8 @@ static void launch_traverse(DeviceObj& D, const char* nm, hipStream_t s, const T
              [&]
              {
                  kern<<<grid, TRAV_BLOCK, 0, s>>>(a.jobs, a.n_jobs, a.q, a.n, a.view, a.hits, a.work, a.chunk,
-                                                 D.xcd_bands == 2 ? 1u : 0u, a.gstack, a.gstride, a.counters);
+                                                 D.xcd_bands == 2 ? 1u : 0u, std::min<uint32_t>(D.trav_refill, 64), a.gstack, a.gstride,
+                                                 a.counters);
              });
     }
 
@@ -572,14 +559,6 @@ template<int SS> static uint32_t max_grid_ss(DeviceObj& D)
                           reinterpret_cast<const void*>(&k_traverse<TRAV_BLOCK, SS, false, true, T_ALL>),
                           reinterpret_cast<const void*>(&k_traverse<TRAV_BLOCK, SS, true, false, T_ALL>),
                           reinterpret_cast<const void*>(&k_traverse<TRAV_BLOCK, SS, true, true, T_ALL>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, false, false, T_SPHERES>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, false, true, T_SPHERES>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, true, false, T_SPHERES>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, true, true, T_SPHERES>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, false, false, T_ALL>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, false, true, T_ALL>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, true, false, T_ALL>),
-                          reinterpret_cast<const void*>(&k_traverse_dyn<TRAV_BLOCK, SS, true, true, T_ALL>),
                           reinterpret_cast<const void*>(&k_traverse_packet<TRAV_BLOCK, SS, false, T_SPHERES>),
                           reinterpret_cast<const void*>(&k_traverse_packet<TRAV_BLOCK, SS, true, T_SPHERES>),
                           reinterpret_cast<const void*>(&k_traverse_packet<TRAV_BLOCK, SS, false, T_ALL>),

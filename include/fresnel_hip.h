@@ -316,13 +316,13 @@ int fh_policy_simulate(uint32_t n, const uint64_t* footprint, const uint64_t* pa
  * rays a batch finishes its paths in one kernel (default 524288); "stack_lds":
  * traversal stack entries kept in LDS per thread, 8 or 16 (default 8);
  * "trav_chunk": rays a secondary-ray traversal wavefront claims per
- * work-counter atomic, a multiple of 64 up to 65536 (default 256);
+ * work-counter atomic, a multiple of 64 up to 65536 (default 256; fewer when
+ * that leaves a wavefront under eight claims, down to 64);
  * "primary_chunk": the most primary rays a primary-kernel workgroup claims at
  * once, a multiple of 64 up to 65536 (default 1024; a batch with fewer than 16
  * such claims per CU claims less, down to 256); "trav_refill": a traversal lane
  * whose ray is done takes a new one once this many lanes of its wavefront are
- * idle, 1..64, or 65 for the batch-synchronous kernel that traces 64 rays at
- * a time (default 65); "trav_packet": primary rays traced as wavefront
+ * idle, 1..64 (65 counts as 64: all lanes; default 32); "trav_packet": primary rays traced as wavefront
  * packets (2, default) or one by one (1); "primary_tiles": primary rays of
  * pinhole-perspective and orthographic cameras tested against per-8x8-tile
  * candidate lists (2, default) or searched in the BVH (1); "tile_min_rays":
