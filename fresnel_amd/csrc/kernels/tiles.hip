@@ -396,6 +396,16 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v)
         p[i] = v;
     }
 
+// Two arrays in one launch.
+__global__ void k_fill2_u32(uint32_t* p, uint32_t n, uint32_t* q, uint32_t m, uint32_t v)
+    {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n)
+        p[i] = v;
+    else if (i - n < m)
+        q[i - n] = v;
+    }
+
 // Sorted entries packed as 8 words each, so a wavefront reads an entry with
 // one scalar load: [0] bound bits, then for spheres-only scenes the sphere
 // (x, y, z, r), geometry slot and primitive, otherwise the box (lo.xyz,

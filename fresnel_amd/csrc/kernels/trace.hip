@@ -799,7 +799,7 @@ __device__ __forceinline__ bool take_view(const QueueView* __restrict__ view, ui
 // view's mode is FINISH when at most `tail` entries are left or `force` is
 // set, BOUNCE for more, IDLE when the queue is empty or a segment overflowed
 // (then CTR_QUEUE_OVERFLOW is raised; the host reports it).  steps[2 step],
-// steps[2 step + 1] record the count and mode.
+// steps[2 step + 1] record the count and mode (pinned host memory).
 __global__ __launch_bounds__(64) void k_queue_view(uint32_t* count, uint32_t seg_cap, uint32_t tail, uint32_t force,
                                                    QueueView* view, uint32_t* work, uint32_t* steps, uint32_t step,
                                                    unsigned long long* counters)
@@ -2307,8 +2307,8 @@ __global__ __launch_bounds__(BLOCK) void k_finish(const JobDev* __restrict__ job
 // ---------------------------------------------------------------- accumulate
 // Replay each camera sample's records in light-sample order, then the Welford
 // mean and sRGB of fresnel/cpu/TracerPath.cc:229-249.
-__global__ void k_accumulate(const JobDev* __restrict__ jobs, const uint32_t* __restrict__ pix_base, uint32_t n_jobs,
-                             uint32_t total, const uint4* __restrict__ records)
+__global__ void k_accumulate(const JobDev* __restrict__ jobs, uint32_t n_jobs, uint32_t total,
+                             const uint4* __restrict__ records)
     {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= total)
@@ -2317,7 +2317,7 @@ __global__ void k_accumulate(const JobDev* __restrict__ jobs, const uint32_t* __
     while (hi - lo > 1)
         {
         const uint32_t mid = (lo + hi) >> 1;
-        if (pix_base[mid] <= i)
+        if (jobs[mid].pix_base <= i)
             lo = mid;
         else
             hi = mid;
@@ -2325,7 +2325,7 @@ __global__ void k_accumulate(const JobDev* __restrict__ jobs, const uint32_t* __
     const JobDev& J = jobs[lo];
     // thread i handles pixel ordinal j (records are chunk-major, so a
     // wavefront reads 64 contiguous records per sample)
-    const uint32_t jord = i - pix_base[lo];
+    const uint32_t jord = i - J.pix_base;
     uint32_t px, py;
     ordinal_pixel(J, jord, px, py);
     const uint32_t pixel = py * J.W + px;

@@ -174,7 +174,7 @@ struct JobDev
     const float4* prim_hi;
     uint32_t tiles_x, tiles_y;
     uint32_t use_tiles;
-    uint32_t pad_tiles;
+    uint32_t pix_base;    // first pixel of this job among the batch's (k_accumulate)
     };
 
 // Termination record of one light-sample path.

@@ -176,9 +176,7 @@ struct RenderScratch
     DBuf<uint2> gstack;        // traversal stack overflow (persistent grid)
     DBuf<uint2> tail_stack;    // stack overflow of the tail kernel
     DBuf<JobDev> jobs;
-    DBuf<uint32_t> pix_base;
     DBuf<QueueView> view;      // consumer view of the queue a bounce step reads (k_queue_view)
-    DBuf<uint32_t> steps;      // count and mode of every bounce step (2 words each)
     };
 
 // Pinned host memory that grows on demand (contents are not preserved).
@@ -297,6 +295,7 @@ struct DeviceObj
     std::vector<hipEvent_t> event_pool;
     std::vector<std::pair<std::string, std::pair<double, uint32_t>>> last_stats;
     uint64_t last_counters[N_CTR] = {};
+    bool counters_zero = false; // the last render left every device counter zero, and nothing ran since
     std::mutex mu;
 
     hipEvent_t event()
@@ -341,9 +340,12 @@ struct DeviceObj
             }
         times.clear();
         counters.ensure(N_CTR);
-        HIPCHECK(hipMemsetAsync(counters.p, 0, N_CTR * sizeof(unsigned long long), stream));
+        if (!counters_zero)
+            HIPCHECK(hipMemsetAsync(counters.p, 0, N_CTR * sizeof(unsigned long long), stream));
+        counters_zero = false;
         }
-    void end_stats()
+    // `ctr`: the counters as the render's batches copied them (nullptr: read here)
+    void end_stats(const unsigned long long* ctr = nullptr)
         {
         HIPCHECK(hipStreamSynchronize(stream));
         if (stream2)
@@ -369,9 +371,16 @@ struct DeviceObj
                 last_stats.push_back({t.name, {ms, 1u}});
             }
         unsigned long long c[N_CTR];
-        HIPCHECK(hipMemcpy(c, counters.p, sizeof(c), hipMemcpyDeviceToHost));
+        if (ctr)
+            std::memcpy(c, ctr, sizeof(c));
+        else
+            HIPCHECK(hipMemcpy(c, counters.p, sizeof(c), hipMemcpyDeviceToHost));
+        counters_zero = true;
         for (int k = 0; k < N_CTR; k++)
+            {
             last_counters[k] = c[k];
+            counters_zero = counters_zero && c[k] == 0;
+            }
         }
     };
 
@@ -656,6 +665,7 @@ struct SceneObj
     std::map<uint32_t, GeometryObj*> geoms; // slot -> geometry
     // device scene
     DBuf<GeomDev> dgeoms;
+    std::vector<GeomDev> table; // dgeoms as last uploaded
     uint32_t n_slots = 0;
     DBuf<float4> blo, bhi;
     DBuf<uint32_t> vals, parent, flags, prefix, slots; // vals: primitive order of the leaves (refit reads it)
@@ -1165,10 +1175,17 @@ static void sync_scene(SceneObj& sc)
         t.aux1 = g.aux1.p;
         t.aux_color = g.daux_color.p;
         }
-    sc.dgeoms.ensure(n_slots);
-    HIPCHECK(hipMemcpyAsync(sc.dgeoms.p, table.data(), n_slots * sizeof(GeomDev), hipMemcpyHostToDevice,
-                            D.copy_stream));
-    uploads_done(D); // before the table goes away and before the device stream's kernels read it
+    // (unchanged since the last upload, byte for byte: it stays)
+    if (table.size() != sc.table.size()
+        || std::memcmp(table.data(), sc.table.data(), table.size() * sizeof(GeomDev)) != 0)
+        {
+        sc.table.clear();
+        sc.dgeoms.ensure(n_slots);
+        HIPCHECK(hipMemcpyAsync(sc.dgeoms.p, table.data(), n_slots * sizeof(GeomDev), hipMemcpyHostToDevice,
+                                D.copy_stream));
+        uploads_done(D); // before the table changes and before the device stream's kernels read it
+        sc.table = table;
+        }
     sc.n_slots = n_slots;
     const bool topo_same = sc.bvh_valid && topo == sc.topo;
     if (!sc.bvh_valid || !topo_same)
@@ -1346,7 +1363,8 @@ struct TracerObj
         finish_copies();
         HIPCHECK(hipMemsetAsync(linear.p, 0, (size_t)W * H * sizeof(float4), dev->stream));
         HIPCHECK(hipMemsetAsync(srgb.p, 0, (size_t)W * H * sizeof(uchar4), dev->stream));
-        HIPCHECK(hipStreamSynchronize(dev->stream));
+        // not waited for: whatever reads or writes the outputs waits for the
+        // device stream (renders by event)
         }
     };
 
@@ -1603,13 +1621,12 @@ static void set_order_divisors(JobDev& J)
     J.div_w = make_fastdiv(std::max(1u, J.W));
     }
 
-// Pinned staging bytes of one batch: its job table, pixel bases and step
-// records (JobDev alignment kept for each part).
+// Pinned staging bytes of one batch: its job table, step records and counters
+// (JobDev alignment kept for each part).
 static size_t stage_bytes(size_t n_jobs)
     {
     auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    return up(n_jobs * sizeof(JobDev)) + up(n_jobs * sizeof(uint32_t)) + up(2 * MAX_STEPS * sizeof(uint32_t))
-           + up(2 * sizeof(unsigned long long));
+    return up(n_jobs * sizeof(JobDev)) + up(2 * MAX_STEPS * sizeof(uint32_t)) + up(N_CTR * sizeof(unsigned long long));
     }
 
 // One batch: every job advances by jobs[j].K camera samples, on one render
@@ -1630,7 +1647,6 @@ struct BatchExec
     std::vector<JobDev> jobs;
     uint32_t types;
     bool spheres;
-    std::vector<uint32_t> pix_base;
     uint64_t n_pri = 0, n_paths = 0, n_pix = 0, n_rec = 0;
     uint32_t nj = 0, gstride = 0, seg_cap = 0, tail_threads = 0, rest_grid = 0, tail_grid = 0;
     uint32_t pgroups = 1; // primary claim size in workgroups of rays (primary_groups)
@@ -1638,8 +1654,8 @@ struct BatchExec
     int cur = 1;
     Queue Q[2];
     uint8_t* stage;
-    uint32_t* h_steps = nullptr; // pinned copy of the step records (valid after the batch has run)
-    unsigned long long* h_flags = nullptr; // pinned copy of the overflow flags after the batch
+    uint32_t* h_steps = nullptr; // pinned step records (valid after the batch has run)
+    unsigned long long* h_ctr = nullptr; // pinned copy of the device counters after the batch
 
     BatchExec(DeviceObj& d, RenderScratch& r, hipStream_t st, std::vector<JobDev> j, uint32_t t, uint8_t* stg)
         : D(d), R(r), s(st), jobs(std::move(j)), types(t), spheres(t == T_SPHERES), stage(stg)
@@ -1651,13 +1667,6 @@ struct BatchExec
         D.lstream = s;
         D.launch(nm, f);
         D.lstream = nullptr;
-        }
-
-    // zero n words with a kernel (no memset node if a caller captures the stream)
-    void clear(uint32_t* p, uint32_t n)
-        {
-        k_fill_u32<<<blocks(n, 256), 256, 0, s>>>(p, n, 0u);
-        HIPCHECK(hipGetLastError());
         }
 
     void traverse(const Queue& q, uint32_t count, const QueueView* view, bool primary)
@@ -1676,7 +1685,7 @@ struct BatchExec
             set_order_divisors(J);
             J.ray_base = (uint32_t)n_pri;
             J.rec_base = n_rec;
-            pix_base.push_back((uint32_t)n_pix);
+            J.pix_base = (uint32_t)n_pix;
             n_pri += (uint64_t)J.npix * J.K;
             n_paths += (uint64_t)J.npix * J.K * J.L;
             n_rec += (uint64_t)((J.npix + 63) / 64) * 64 * J.K * J.L; // whole 64-pixel chunks
@@ -1698,10 +1707,9 @@ struct BatchExec
         gstride = D.trav_grid * TRAV_BLOCK; // max resident threads of any traversal variant
         tail_threads = blocks(D.tail_rays, TRAV_BLOCK) * TRAV_BLOCK;
         const bool fits = R.hits.cap >= std::max(n_pri, n_paths) && R.qo[0].cap >= cap && R.qo[1].cap >= cap
-                          && R.records.cap >= n_rec && R.jobs.cap >= jobs.size() && R.pix_base.cap >= jobs.size()
+                          && R.records.cap >= n_rec && R.jobs.cap >= jobs.size()
                           && R.gstack.cap >= (size_t)(STACK_MAX - 8) * gstride
-                          && R.tail_stack.cap >= (size_t)(STACK_MAX - TRAV_SS) * tail_threads && R.view.p && R.steps.p
-                          && R.counters32.p && R.qseg.p;
+                          && R.tail_stack.cap >= (size_t)(STACK_MAX - TRAV_SS) * tail_threads && R.view.p && R.counters32.p && R.qseg.p;
         if (!fits)
             HIPCHECK(hipStreamSynchronize(s));
         R.hits.ensure(std::max(n_pri, n_paths));
@@ -1716,21 +1724,17 @@ struct BatchExec
         R.counters32.ensure(8 * QSEG_STRIDE);
         R.qseg.ensure(QSEG_FLAG + 1);
         R.jobs.ensure(jobs.size());
-        R.pix_base.ensure(jobs.size());
         R.view.ensure(1);
-        R.steps.ensure(2 * MAX_STEPS);
-        // job table and pixel bases through pinned staging: the copies do not
-        // wait for the stream, so enqueueing never blocks on earlier batches
+        // job table through pinned staging: the copy does not wait for the
+        // stream, so enqueueing never blocks on earlier batches; the step
+        // records are written to the staging by k_queue_view itself
         uint8_t* p = stage;
         std::memcpy(p, jobs.data(), jobs.size() * sizeof(JobDev));
         HIPCHECK(hipMemcpyAsync(R.jobs.p, p, jobs.size() * sizeof(JobDev), hipMemcpyHostToDevice, s));
         p += (jobs.size() * sizeof(JobDev) + 255) & ~(size_t)255;
-        std::memcpy(p, pix_base.data(), pix_base.size() * 4);
-        HIPCHECK(hipMemcpyAsync(R.pix_base.p, p, pix_base.size() * 4, hipMemcpyHostToDevice, s));
-        p += (pix_base.size() * 4 + 255) & ~(size_t)255;
         h_steps = (uint32_t*)p;
         p += (2 * MAX_STEPS * sizeof(uint32_t) + 255) & ~(size_t)255;
-        h_flags = (unsigned long long*)p;
+        h_ctr = (unsigned long long*)p;
         R.gstack.ensure((size_t)(STACK_MAX - 8) * gstride);
         // the tail kernel's grid-stride threads (at least tail_rays)
         R.tail_stack.ensure((size_t)(STACK_MAX - TRAV_SS) * tail_threads);
@@ -1786,8 +1790,8 @@ struct BatchExec
                               (const void*)R.qd[1].p, (const void*)R.qatt[0].p, (const void*)R.qatt[1].p,
                               (const void*)R.qmeta[0].p, (const void*)R.qmeta[1].p, (const void*)R.hits.p,
                               (const void*)R.records.p, (const void*)R.counters32.p, (const void*)R.qseg.p,
-                              (const void*)R.jobs.p, (const void*)R.pix_base.p, (const void*)R.view.p,
-                              (const void*)R.steps.p, (const void*)R.gstack.p, (const void*)R.tail_stack.p,
+                              (const void*)R.jobs.p, (const void*)R.view.p,
+                              (const void*)h_steps, (const void*)R.gstack.p, (const void*)R.tail_stack.p,
                               (const void*)D.counters.p})
             k.push_back((uint64_t)(uintptr_t)p);
         for (uint32_t b = 0; b < steps; b++)
@@ -1799,8 +1803,9 @@ struct BatchExec
     void enqueue_kernels(uint32_t steps)
         {
         const uint32_t groups = pgroups;
-        clear(R.counters32.p, 8 * QSEG_STRIDE);
-        clear(R.qseg.p, QSEG_FLAG + 1);
+        k_fill2_u32<<<blocks(8 * QSEG_STRIDE + QSEG_FLAG + 1, 256), 256, 0, s>>>(R.counters32.p, 8 * QSEG_STRIDE,
+                                                                                R.qseg.p, QSEG_FLAG + 1, 0u);
+        HIPCHECK(hipGetLastError());
         if (D.fuse_primary == 2)
             {
             PrimaryArgs a {R.jobs.p, nj, (uint32_t)n_pri, R.counters32.p, groups, R.gstack.p, gstride, Q[1],
@@ -1824,10 +1829,19 @@ struct BatchExec
         enqueue_steps(steps);
         }
 
+    // Whether every path fits the tail kernel: the first step's view then selects
+    // it whatever the queue holds, and nothing else needs enqueueing.
+    bool tail_only() const
+        {
+        return n_paths <= D.tail_rays;
+        }
+
     // Enqueue `steps` bounce steps (1 <= steps <= MAX_STEPS); the last one
     // finishes every path that is still queued.
     void enqueue_steps(uint32_t steps)
         {
+        if (tail_only())
+            steps = 1;
         auto* f = finish_kernel();
         auto* shade_one = spheres ? k_shade<SHADE_BLOCK, T_SPHERES, false> : k_shade<SHADE_BLOCK, T_ALL, false>;
         auto* shade_rest = spheres ? k_shade<SHADE_BLOCK, T_SPHERES, true> : k_shade<SHADE_BLOCK, T_ALL, true>;
@@ -1839,12 +1853,15 @@ struct BatchExec
                    [&]
                    {
                        k_queue_view<<<1, 64, 0, s>>>(R.qseg.p, seg_cap, D.tail_rays, last ? 1u : 0u, R.view.p,
-                                                     R.counters32.p, R.steps.p, b, D.counters.p);
+                                                     R.counters32.p, h_steps, b, D.counters.p);
                    });
             const Queue in = Q[cur], out = Q[1 - cur];
             D.tag_mode = mode;
             D.tag_acts_on = VIEW_BOUNCE;
-            if (D.fuse_bounce == 2)
+            if (tail_only())
+                {
+                }
+            else if (D.fuse_bounce == 2)
                 {
                 BounceArgs a {R.jobs.p, in, 0u, R.view.p, R.counters32.p, D.trav_chunk, R.gstack.p, gstride, out,
                               R.records.p, D.counters.p};
@@ -1889,18 +1906,16 @@ struct BatchExec
         n_steps = steps;
         }
 
-    // Copy the step records and the device's overflow flags (queue segment,
-    // traversal stack) to the pinned staging, after the steps.
-    void copy_steps()
+    // Copy the device counters (overflow flags among them) to the pinned
+    // staging, after the steps.
+    void copy_counters()
         {
-        HIPCHECK(hipMemcpyAsync(h_steps, R.steps.p, 2 * n_steps * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        HIPCHECK(hipMemcpyAsync(h_flags, D.counters.p + CTR_QUEUE_OVERFLOW, 2 * sizeof(unsigned long long),
-                                hipMemcpyDeviceToHost, s));
+        HIPCHECK(hipMemcpyAsync(h_ctr, D.counters.p, N_CTR * sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
         }
 
     // The batch's kernels, launched or (D.graph == 2 and no per-launch timing
     // or counting) captured once per key into a HIP graph and replayed; then
-    // the step records' copy.  The job table copies (start) and the
+    // the counters' copy.  The job table copies (start) and the
     // accumulation, which waits on another stream's event, stay outside the
     // graph, as no memset is inside it.
     void run(uint32_t steps)
@@ -1908,7 +1923,7 @@ struct BatchExec
         if (D.graph != 2 || D.stats_on || D.count_on)
             {
             enqueue_kernels(steps);
-            copy_steps();
+            copy_counters();
             return;
             }
         const std::vector<uint64_t> key = graph_key(steps);
@@ -1945,9 +1960,9 @@ struct BatchExec
             D.graph_captures++;
             }
         else
-            n_steps = steps; // as enqueue_kernels sets it
+            n_steps = tail_only() ? 1 : steps; // as enqueue_kernels sets it
         HIPCHECK(hipGraphLaunch(exec, s));
-        copy_steps();
+        copy_counters();
         }
 
     // Fold this batch's queued fraction at each bounce step into the device's
@@ -1983,7 +1998,7 @@ struct BatchExec
         launch("accumulate",
                [&]
                {
-                   k_accumulate<<<blocks(n_pix, 256), 256, 0, s>>>(R.jobs.p, R.pix_base.p, nj, (uint32_t)n_pix,
+                   k_accumulate<<<blocks(n_pix, 256), 256, 0, s>>>(R.jobs.p, nj, (uint32_t)n_pix,
                                                                    R.records.p);
                });
         if (done)
@@ -2050,6 +2065,9 @@ struct InflightRun
     int slot = 0;
     size_t off = 0;
     uint32_t steps = 0;
+    // the device counters after finish(): they only grow, so the largest of the
+    // batches' copies
+    unsigned long long ctr[N_CTR] = {};
 
     // `stage` bytes of pinned staging for the job tables of every batch to come
     InflightRun(DeviceObj& d, size_t stage) : D(d)
@@ -2090,19 +2108,26 @@ struct InflightRun
         {
         HIPCHECK(hipStreamSynchronize(D.stream3));
         HIPCHECK(hipStreamSynchronize(D.stream2));
-        uint32_t need = 1;
+        uint32_t need = 0;
         float live[MAX_STEPS] = {};
         for (const auto& e : batches)
             {
+            for (int k = 0; k < N_CTR; k++)
+                ctr[k] = std::max<unsigned long long>(ctr[k], e->h_ctr[k]);
+            if (e->tail_only())
+                continue; // says nothing about the bounce steps of larger batches
             need = std::max(need, e->steps_needed());
             e->note_live(live);
             }
+        if (need == 0)
+            return;
         update_steps_est(D, need);
         update_live_frac(D, live);
         }
     };
 
-static void run_inflight(DeviceObj& D, std::deque<std::pair<std::vector<JobDev>, uint32_t>>& pending)
+static void run_inflight(DeviceObj& D, std::deque<std::pair<std::vector<JobDev>, uint32_t>>& pending,
+                         unsigned long long* ctr)
     {
     size_t bytes = 0;
     for (const auto& b : pending)
@@ -2114,6 +2139,7 @@ static void run_inflight(DeviceObj& D, std::deque<std::pair<std::vector<JobDev>,
         pending.pop_front();
         }
     run.finish();
+    std::memcpy(ctr, run.ctr, sizeof(run.ctr));
     }
 
 // Render `samples` Path passes for each (scene, tracer) pair.
@@ -2127,6 +2153,7 @@ static void render_path(DeviceObj& D, const std::vector<SceneObj*>& scenes, cons
         REQUIRE(scenes[k]->dev == tracers[k]->dev, "Scene and Tracer devices do not match");
         REQUIRE(tracers[k]->type == T_PATH, "not a Path tracer");
         }
+    unsigned long long ctr[N_CTR] = {};
     uint64_t per_sample = 0;
     for (auto* tr : tracers)
         per_sample += (uint64_t)tr->W * tr->H * tr->L;
@@ -2199,6 +2226,7 @@ static void render_path(DeviceObj& D, const std::vector<SceneObj*>& scenes, cons
                 run.add(std::move(g.first), g.second);
             }
         run.finish();
+        std::memcpy(ctr, run.ctr, sizeof(ctr));
         }
     else
         {
@@ -2230,11 +2258,11 @@ static void render_path(DeviceObj& D, const std::vector<SceneObj*>& scenes, cons
             split_groups(jobs, types, groups);
             done += k;
             }
-        run_inflight(D, groups);
+        run_inflight(D, groups, ctr);
         }
     for (auto* tr : tracers)
         tr->n_samples += samples;
-    D.end_stats();
+    D.end_stats(ctr);
     if (D.last_counters[CTR_OVERFLOW])
         throw Error(FH_ERR_STATE, "traversal stack overflow");
     }
@@ -2259,7 +2287,10 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     tr.order_after_copies(D.stream, nullptr);
     RenderScratch& R = D.rs;
     R.jobs.ensure(1);
-    HIPCHECK(hipMemcpyAsync(R.jobs.p, &J, sizeof(J), hipMemcpyHostToDevice, D.stream));
+    D.stage.ensure(stage_bytes(1));
+    std::memcpy(D.stage.p, &J, sizeof(J));
+    HIPCHECK(hipMemcpyAsync(R.jobs.p, D.stage.p, sizeof(J), hipMemcpyHostToDevice, D.stream));
+    unsigned long long* ctr = (unsigned long long*)(D.stage.p + stage_bytes(1) - 256);
     // with at least as many samples as a workgroup has wavefronts they share
     // one chunk of 64 pixels, else each takes its own
     const bool split = (uint64_t)tr.aa_n * tr.aa_n >= PREVIEW_BLOCK / 64;
@@ -2274,7 +2305,9 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     D.launch("preview",
              [&] { kern<<<grid, PREVIEW_BLOCK, 0, D.stream>>>(R.jobs.p, tr.aa_n, own_search ? 1u : 0u, R.gstack.p,
                                                          gstride, D.counters.p); });
-    D.end_stats();
+    HIPCHECK(hipMemcpyAsync(ctr, D.counters.p, N_CTR * sizeof(*ctr), hipMemcpyDeviceToHost, D.stream));
+    HIPCHECK(hipStreamSynchronize(D.stream));
+    D.end_stats(ctr);
     if (D.last_counters[CTR_OVERFLOW])
         throw Error(FH_ERR_STATE, "traversal stack overflow");
     }
@@ -2546,11 +2579,14 @@ static void server_finish_batch(ServerObj& S, size_t i)
     {
     DeviceObj& D = *S.dev;
     ServerBatch& b = S.batches[i];
-    update_steps_est(D, b.e->steps_needed());
-    float live[MAX_STEPS] = {};
-    b.e->note_live(live);
-    update_live_frac(D, live);
-    const unsigned long long q_flag = b.e->h_flags[0], s_flag = b.e->h_flags[1];
+    if (!b.e->tail_only())
+        {
+        update_steps_est(D, b.e->steps_needed());
+        float live[MAX_STEPS] = {};
+        b.e->note_live(live);
+        update_live_frac(D, live);
+        }
+    const unsigned long long q_flag = b.e->h_ctr[CTR_QUEUE_OVERFLOW], s_flag = b.e->h_ctr[CTR_OVERFLOW];
     for (auto& a : b.adds)
         S.reqs[a.first].done += a.second;
     const int kd = b.kind();
@@ -2713,9 +2749,10 @@ static void server_step(ServerObj& S, double now, uint32_t& n_active, uint32_t& 
                 }
             b.stage->ensure(stage_bytes(b.jobs.size()));
             b.e.reset(new BatchExec(D, S.rs[k], S.st[k], b.jobs, b.types, b.stage->p));
+            D.counters_zero = false;
             b.e->start();
             b.e->enqueue_kernels(D.steps_est);
-            b.e->copy_steps();
+            b.e->copy_counters();
             b.done = S.free_events.back();
             const int kd = b.kind();
             b.e->accumulate(S.last_acc[kd], b.done);
@@ -3607,6 +3644,7 @@ extern "C"
                 NONNULL(data);
                 TracerObj& T = tr->obj;
                 const size_t n = (size_t)T.W * T.H;
+                HIPCHECK(hipStreamSynchronize(T.dev->stream)); // a clear may still be queued
                 if (which == FH_OUT_SRGB)
                     {
                     HIPCHECK(hipMemcpy(T.h_srgb.data(), T.srgb.p, n * 4, hipMemcpyDeviceToHost));

@@ -1,0 +1,69 @@
+"""Repeated renders of one scene and tracer: what a call leaves out must not show."""
+
+import numpy
+import pytest
+
+import fresnel_amd as fresnel
+from test_gpu_parity import c1_scene
+
+pytestmark = pytest.mark.gpu
+
+
+def test_outputs_read_after_reset_are_clear(gpu_device):
+    """reset() queues the clearing of the outputs; every way of reading them waits for it."""
+    s = c1_scene(gpu_device, n=300)
+    t = fresnel.tracer.Path(gpu_device, w=640, h=480)
+    for _ in range(5):
+        t.sample(s, samples=2)
+        assert t.linear_output[:].any()
+        t.reset()
+        assert not t.linear_output[:].any()
+        t.sample(s, samples=2)
+        t.reset()
+        assert not t.output[:].any()
+        t.sample(s, samples=2)
+        t.reset()
+        assert not numpy.array(t.output_async(linear=True).wait()).any()
+        assert t.histogram()[0].sum() == 0
+
+
+@pytest.mark.parametrize('tracer', ['Path', 'Preview'])
+def test_material_changes_between_renders(tracer, gpu_device):
+    """The geometry table is uploaded again when anything in it changed, and only then."""
+    s = c1_scene(gpu_device, n=300)
+    colors = [(0.9, 0.1, 0.1), (0.1, 0.9, 0.1), (0.1, 0.9, 0.1), (0.9, 0.1, 0.1)]
+    images = []
+    t = getattr(fresnel.tracer, tracer)(gpu_device, w=96, h=64)
+    for c in colors:
+        s.geometry[0].material.color = c
+        t.seed = 5
+        if tracer == 'Path':
+            t.sample(s, samples=2)
+        else:
+            t.render(s)
+        images.append(numpy.array(t.linear_output[:]))
+    assert numpy.array_equal(images[1], images[2])
+    assert numpy.array_equal(images[0], images[3])
+    assert not numpy.array_equal(images[0], images[1])
+    s.geometry[0].outline_width = 0.3
+    t.seed = 5
+    t.sample(s, samples=2) if tracer == 'Path' else t.render(s)
+    assert not numpy.array_equal(images[3], t.linear_output[:])
+
+
+@pytest.mark.parametrize('tail_rays', [96 * 64 * 3 - 1, 96 * 64 * 3, 96 * 64 * 3 + 1])
+def test_tail_only_batches(tail_rays, gpu_device):
+    """A batch of exactly, just under and just over tail_rays paths: the same image."""
+    s = c1_scene(gpu_device, n=3000)
+    t = fresnel.tracer.Path(gpu_device, w=96, h=64)
+    t.seed = 5
+    t.sample(s, samples=3)
+    ref = numpy.array(t.linear_output[:])
+    old = gpu_device._device.tune('tail_rays', tail_rays)
+    try:
+        for _ in range(2):
+            t.seed = 5
+            t.sample(s, samples=3)
+            numpy.testing.assert_array_equal(t.linear_output[:], ref)
+    finally:
+        gpu_device._device.tune('tail_rays', old)
