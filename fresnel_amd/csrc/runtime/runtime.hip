@@ -399,12 +399,13 @@ struct TravArgs
     uint2* gstack;
     uint32_t gstride;
     unsigned long long* counters;
+    bool per_ray = false; // primary rays: search each on its own whatever trav_packet says
     };
 
 template<int SS, bool C, bool P, uint32_t T>
 static void launch_traverse(DeviceObj& D, const char* nm, hipStream_t s, const TravArgs& a)
     {
-    if (P && D.trav_packet == 2)
+    if (P && D.trav_packet == 2 && !a.per_ray)
         {
         auto kern = &k_traverse_packet<TRAV_BLOCK, SS, C, T>;
         const uint32_t grid = D.grid_for(reinterpret_cast<const void*>(kern), TRAV_BLOCK);
@@ -1672,7 +1673,7 @@ struct BatchExec
     void traverse(const Queue& q, uint32_t count, const QueueView* view, bool primary)
         {
         TravArgs a {R.jobs.p, nj, q, count, view, R.hits.p, R.counters32.p, D.trav_chunk, R.gstack.p, gstride,
-                    D.counters.p};
+                    D.counters.p, primary && per_ray_primary()};
         D.lstream = s;
         dispatch_traverse(D, primary ? "traverse_primary" : "traverse", s, a, primary, spheres);
         D.lstream = nullptr;
@@ -1785,7 +1786,8 @@ struct BatchExec
         std::vector<uint64_t> k = {(uint64_t)(uintptr_t)s, nj, n_pri, n_paths, n_pix, n_rec, seg_cap, gstride,
                                    tail_threads, types, steps, D.trav_chunk, pgroups, D.xcd_bands,
                                    D.fuse_primary, D.fuse_bounce, D.tail_rays, (uint64_t)D.stack_lds, D.trav_refill,
-                                   D.trav_packet, D.count_on ? 1u : 0u, rest_grid, tail_grid};
+                                   D.trav_packet, D.count_on ? 1u : 0u, rest_grid, tail_grid,
+                                   per_ray_primary() ? 1u : 0u};
         for (const void* p : {(const void*)R.qo[0].p, (const void*)R.qo[1].p, (const void*)R.qd[0].p,
                               (const void*)R.qd[1].p, (const void*)R.qatt[0].p, (const void*)R.qatt[1].p,
                               (const void*)R.qmeta[0].p, (const void*)R.qmeta[1].p, (const void*)R.hits.p,
@@ -1799,6 +1801,36 @@ struct BatchExec
         return k;
         }
 
+    // Whether the primary rays are searched one by one (k_traverse, lanes
+    // refilled) instead of as packets of a tile, fused with their shading
+    // (k_primary), when neither knob asks for a form of its own.  Packets walk
+    // the binary tree once for 64 rays, which pays while a tile's rays meet the
+    // same few primitives; with many small ones per tile most of a packet's
+    // visits serve few lanes.  Measured (packets / per ray, ms of primary
+    // rays): spherocylinders, 853 x 480, 16 samples, at 0.6, 2.5 and 10
+    // primitives per 64 pixels 0.98 / 1.17, 1.70 / 1.27, 2.44 / 1.48; mesh
+    // triangles at 2, 8 and 32 0.91 / 1.08, 1.61 / 1.22, 2.47 / 1.41; at 256 x
+    // 256, 8 samples, whose few rays leave the separate kernels idle longer,
+    // spherocylinders at 3.9, 16 and 63 0.26 / 0.38, 0.44 / 0.46, 0.70 / 0.56,
+    // triangles at 13, 50 and 200 0.33 / 0.37, 0.47 / 0.45, 0.86 / 0.58.
+    // Spheres stay with packets (their test is the cheapest: 1.56 / 1.62 at
+    // 78), as do tile lists, and scenes with polyhedra, whose grazing faces
+    // make a hit depend on the search's order (k_preview).
+    bool per_ray_primary() const
+        {
+        if (spheres || (types & (1u << G_POLYHEDRON)) || D.fuse_primary != 2 || D.trav_packet != 2)
+            return false;
+        uint64_t prims = 0;
+        for (const auto& J : jobs)
+            {
+            if (J.use_tiles)
+                return false;
+            prims += J.scene.n_prims;
+            }
+        const double per_tile = 64.0 * (double)prims / (double)std::max<uint64_t>(n_pix, 1);
+        return per_tile * (double)std::min<uint64_t>(n_pri, 4ull << 20) >= (double)(16ull << 20);
+        }
+
     // The batch's kernels: counter clears, primary rays, `steps` bounce steps.
     void enqueue_kernels(uint32_t steps)
         {
@@ -1806,7 +1838,7 @@ struct BatchExec
         k_fill2_u32<<<blocks(8 * QSEG_STRIDE + QSEG_FLAG + 1, 256), 256, 0, s>>>(R.counters32.p, 8 * QSEG_STRIDE,
                                                                                 R.qseg.p, QSEG_FLAG + 1, 0u);
         HIPCHECK(hipGetLastError());
-        if (D.fuse_primary == 2)
+        if (D.fuse_primary == 2 && !per_ray_primary())
             {
             PrimaryArgs a {R.jobs.p, nj, (uint32_t)n_pri, R.counters32.p, groups, R.gstack.p, gstride, Q[1],
                            R.records.p, D.counters.p};
