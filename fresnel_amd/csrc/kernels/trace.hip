@@ -2460,8 +2460,12 @@ __device__ __forceinline__ float4 preview_shade(const JobDev& J, const HitT& h, 
 // 64 serial samples, in raster order with the stack in scratch, took 5.99 ms
 // for 500 spheres at 600 x 370 and 34.3 ms for 20,000 polyhedra at 1280 x
 // 720, 64 samples each, image read included; this form takes 0.67 and 16.8 ms.
+// Held to 80 registers (6 wavefronts per SIMD, what the LDS allows; some values
+// spill): 1280 x 720, 64 samples of 500 spheres 0.69 -> 0.62 ms of kernel,
+// 20,000 spherocylinders 2.8 -> 2.5, 500 meshes 6.4 -> 5.6, mixed 17.8 -> 16.2
+// against the 4 that 113 to 127 registers allow.
 template<int BLOCK, int SS, uint32_t TYPES, bool SPLIT>
-__global__ __launch_bounds__(BLOCK) void k_preview(const JobDev* __restrict__ jobp, uint32_t aa_n,
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_preview(const JobDev* __restrict__ jobp, uint32_t aa_n,
                                                    uint32_t own_search, uint2* gstack, uint32_t gstride,
                                                    unsigned long long* counters)
     {
