@@ -15,9 +15,8 @@ the timed region).  Mpaths/s = W*H*samples*light_samples per second.  The
 JSON line also carries:
   roofline         the kernel with the most time per frame (the
                    secondary-ray traversal or the fused primary kernel):
-                   algorithmic bytes per launch (128 B per 4-wide node visit
-                   of a spheres-only hierarchy, 64 B per binary node visit,
-                   prim_bytes per primitive tested, the ray's own bytes, from
+                   algorithmic bytes per launch (64 B per hierarchy node visit,
+                   4-wide or binary, prim_bytes per primitive tested, the ray's own bytes, from
                    the instrumented work counters) over the average launch
                    duration (HIP events on the stream it runs on), against
                    8 TB/s HBM; beside it the same launches' model FP32 flops
@@ -74,11 +73,12 @@ if ROOT not in sys.path:
 METRIC = "Mpaths/s + p50/p99 frame latency, served/batched vs plain, at fixed image RMSE"
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3
-# Model FP32 operations of the traversal: a child box slab test (3 axes x
-# (2 subtractions + 2 multiplications) + 4 min/max + the cull bound) ~20, so
-# 80 per 4-wide node visit (4 children) and 40 per binary node visit (2);
-# a sphere test (centre offset, two dot products, discriminant, root) ~20; a
-# ray's setup (3 reciprocals, 3 multiplications) ~6.
+# Model FP32 operations of the searches: a child box slab test ~20 (3 axes x
+# two fmas and the cull bound in the 4-wide search, 3 axes x (2 subtractions +
+# 2 multiplications) and more in the binary one), so 80 per 4-wide node visit
+# (4 children) and 40 per binary node visit (2); a sphere test (centre offset,
+# two dot products, discriminant, root) ~20; a ray's setup (3 reciprocals, 3
+# multiplications) ~6.
 FLOPS_PER_NODE4, FLOPS_PER_NODE2, FLOPS_PER_SPHERE, FLOPS_PER_RAY = 80, 40, 20, 6
 
 
@@ -241,15 +241,15 @@ def c3_scene(device, a=None, n_poly=200000, n_cyl=2000000, n_mesh=50000, side=12
 
 
 WORKLOADS = {
-    'c2': dict(build=c2_scene, arrays=c2_arrays, W=1920, H=1080, samples=256, light_samples=1, prim_bytes=16, node_bytes=128,
+    'c2': dict(build=c2_scene, arrays=c2_arrays, W=1920, H=1080, samples=256, light_samples=1, prim_bytes=16,
                name="1,048,576 spheres, 64^3 FCC lattice a=1.5 jitter 0.05, r~U[0.4,0.6], HSV colors, "
                "roughness 0.3 specular 0.5, outline 0.05, light.cloudy(), perspective fit; "
                "1920x1080, samples=256, light_samples=1"),
-    'c1': dict(build=c1_scene, arrays=c1_arrays, W=256, H=256, samples=16, light_samples=8, prim_bytes=16, node_bytes=128,
+    'c1': dict(build=c1_scene, arrays=c1_arrays, W=256, H=256, samples=16, light_samples=8, prim_bytes=16,
                name="4096 spheres uniform in a cube of side 20 (seed 0), r=0.5, outline 0.1, "
                "color linear(0.1,0.8,0.1) roughness 0.8 specular 0.2, light.cloudy(), perspective fit; "
                "256x256, samples=16, light_samples=8"),
-    'c3': dict(build=c3_scene, arrays=c3_arrays, W=1920, H=1080, samples=128, light_samples=1, prim_bytes=28, node_bytes=64,
+    'c3': dict(build=c3_scene, arrays=c3_arrays, W=1920, H=1080, samples=128, light_samples=1, prim_bytes=28,
                name="200k cuboid polyhedra 1x1x0.5 random orientations + 2M spherocylinders r=0.1 joining "
                "1st/2nd nearest neighbours of 1M points + 50k icosphere meshes (320 triangles, r=0.4), "
                "cube of side 120, materials rough 0.1/0.5/0.9 metal 0/1/0, light.cloudy(), perspective fit; "
@@ -412,8 +412,9 @@ def run_plain(args):
         valu_busy = prof.get('valu_busy_pct', {})
         valu_lanes = prof.get('valu_active_lanes_pct', {})
 
-    node_bytes = wl.get('node_bytes', 64)
-    flops_node = FLOPS_PER_NODE4 if node_bytes == 128 else FLOPS_PER_NODE2
+    # 64-byte nodes: 4-wide in the secondary and tail searches, binary in the
+    # primary packets and list subtrees
+    node_bytes = 64
 
     def kernel_roofline(name, rays, nodes, prims, ray_bytes, what):
         """Algorithmic bytes per launch (node_bytes per hierarchy node visited, prim_bytes per
@@ -424,6 +425,7 @@ def run_plain(args):
         launches = max(1, kstats[-1].get(name, (0.0, 1))[1])
         alg = node_bytes * nodes + pb * prims + ray_bytes * rays
         achieved = alg / (ms / 1e3) / 1e9 if ms > 0 else 0.0
+        flops_node = FLOPS_PER_NODE2 if name == 'primary' else FLOPS_PER_NODE4
         flops = flops_node * nodes + FLOPS_PER_SPHERE * prims + FLOPS_PER_RAY * rays
         tflops = flops / (ms / 1e3) / 1e12 if ms > 0 else 0.0
         t = traffic.get(name)
@@ -462,8 +464,9 @@ def run_plain(args):
                 "binding": binding}
 
     # primary rays are generated in the kernel; the fused primary kernel
-    # (k_primary) writes at least a 16 B record or queue entry per ray, the
-    # unfused one a 16 B hit.  Secondary rays read 32 B of ray from the queue
+    # (k_primary) writes at least a 16 B record or queue entry per ray of a
+    # tile that lists anything (background tiles are skipped), the unfused one
+    # a 16 B hit.  Secondary rays read 32 B of ray from the queue
     # and write a 16 B hit.
     primary_name = "primary" if "primary" in kstats[-1] else "traverse_primary"
     roof = {primary_name: kernel_roofline(primary_name, ctr[3], ctr[4], ctr[5], 16,
@@ -478,7 +481,7 @@ def run_plain(args):
     seg_rays = ctr[0] + ctr[3] + ctr[6]
     path_bytes = (node_bytes * (ctr[1] + ctr[4] + ctr[7]) + pb * (ctr[2] + ctr[5] + ctr[8])
                   + 36 * W * H * S)
-    path_flops = (flops_node * (ctr[1] + ctr[4] + ctr[7]) + FLOPS_PER_SPHERE * (ctr[2] + ctr[5] + ctr[8])
+    path_flops = (FLOPS_PER_NODE4 * (ctr[1] + ctr[7]) + FLOPS_PER_NODE2 * ctr[4] + FLOPS_PER_SPHERE * (ctr[2] + ctr[5] + ctr[8])
                   + FLOPS_PER_RAY * seg_rays)
     kernel_ms = {k: round(v[0], 3) for k, v in kstats[-1].items()}
     kernel_launches = {k: int(v[1]) for k, v in kstats[-1].items()}
