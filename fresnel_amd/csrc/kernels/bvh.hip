@@ -481,7 +481,8 @@ __global__ void k_refit(const uint32_t* __restrict__ vals, const float4* __restr
 // The binary hierarchy's inner nodes at even depth become the nodes of a
 // 4-wide hierarchy whose children are their grandchildren (a child that is a
 // leaf stays a child), so a search makes half as many dependent node fetches.
-// The binary tree is the one built and refit; the 4-wide nodes copy its boxes
+// The binary tree is the one built and refit; the 4-wide nodes hold its boxes
+// rounded outwards
 // (k_bvh4_fill after every build and refit, the topology from k_depth_even and
 // a scan of its flags).
 

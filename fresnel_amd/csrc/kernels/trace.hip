@@ -201,8 +201,9 @@ struct TraceState
     };
 
 // One node visit of the closest-hit search over the binary hierarchy (the
-// subtrees of tile lists): the primitives of leaf children are tested, the nearer hit inner child is visited next and the farther one
-// pushed.  Returns false when the search is complete.  The closest hit is
+// subtrees of tile lists): the primitives of leaf children are tested, the
+// nearer hit inner child is visited next and the farther one pushed.  Returns
+// false when the search is complete.  The closest hit is
 // the smallest (t, geometry, primitive) over the primitives whose bounds pass
 // the slab test with tmax >= tnear; a subtree is culled when the lower bound
 // of its primitives' distances (cull_bound) exceeds the closest hit.
