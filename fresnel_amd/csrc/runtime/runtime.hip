@@ -234,6 +234,7 @@ struct DeviceObj
     hipStream_t stream3 = nullptr; // first render stream (`stream` builds scenes and tile lists)
     hipStream_t copy_stream = nullptr; // asynchronous output readback; scene uploads
     hipEvent_t upload_ev = nullptr;    // end of the scene uploads queued on copy_stream
+    bool uploads_queued = false;       // scene uploads on copy_stream that uploads_done has not ordered yet
     hipEvent_t build_ev = nullptr;     // device-stream work a render batch waits for (InflightRun)
     hipStream_t lstream = nullptr; // stream of the launches being enqueued (timing events)
     int n_cu = 0;
@@ -932,6 +933,7 @@ static void uploads_done(DeviceObj& D)
     HIPCHECK(hipEventRecord(D.upload_ev, D.copy_stream));
     HIPCHECK(hipStreamWaitEvent(D.stream, D.upload_ev, 0));
     HIPCHECK(hipEventSynchronize(D.upload_ev));
+    D.uploads_queued = false;
     }
 
 // The traversal's cull margin, CULL_K * 3 * the largest primitive half-extent,
@@ -1142,6 +1144,7 @@ static void sync_scene(SceneObj& sc)
         if (g.dirty || g.shape_hi > g.shape_lo || g.color_hi > g.color_lo)
             {
             // colour-only changes leave the hierarchy as it is
+            D.uploads_queued = true;
             if (upload_geometry(g, D.copy_stream) && g.enabled)
                 any_dirty = true;
             }
@@ -1177,16 +1180,23 @@ static void sync_scene(SceneObj& sc)
         t.aux_color = g.daux_color.p;
         }
     // (unchanged since the last upload, byte for byte: it stays)
-    if (table.size() != sc.table.size()
-        || std::memcmp(table.data(), sc.table.data(), table.size() * sizeof(GeomDev)) != 0)
+    const bool changed = table.size() != sc.table.size()
+                         || std::memcmp(table.data(), sc.table.data(), table.size() * sizeof(GeomDev)) != 0;
+    if (changed)
         {
         sc.table.clear();
         sc.dgeoms.ensure(n_slots);
+        D.uploads_queued = true;
         HIPCHECK(hipMemcpyAsync(sc.dgeoms.p, table.data(), n_slots * sizeof(GeomDev), hipMemcpyHostToDevice,
                                 D.copy_stream));
-        uploads_done(D); // before the table changes and before the device stream's kernels read it
-        sc.table = table;
         }
+    // before the table and the colour buffers change and before the device
+    // stream's kernels read them; a colour edit uploads rows without a new
+    // table or hierarchy
+    if (D.uploads_queued)
+        uploads_done(D);
+    if (changed)
+        sc.table = std::move(table);
     sc.n_slots = n_slots;
     const bool topo_same = sc.bvh_valid && topo == sc.topo;
     if (!sc.bvh_valid || !topo_same)

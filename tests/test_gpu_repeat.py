@@ -67,3 +67,41 @@ def test_tail_only_batches(tail_rays, gpu_device):
             numpy.testing.assert_array_equal(t.linear_output[:], ref)
     finally:
         gpu_device._device.tune('tail_rays', old)
+
+
+@pytest.mark.parametrize('tracer', ['Path', 'Preview'])
+def test_color_edits_reach_the_next_render(tracer, gpu_device):
+    """All colors of a large unchanged scene rewritten before every render (12 MB of copies, no new table or hierarchy):
+    each image is that of a scene built with those colors."""
+    n = 1 << 20
+    rng = numpy.random.default_rng(4)
+    pos = rng.uniform(-40, 40, (n, 3)).astype(numpy.float32)
+    colors = [rng.uniform(0, 1, (n, 3)).astype(numpy.float32) for _ in range(2)]
+
+    def build(c):
+        s = fresnel.Scene(gpu_device, lights=fresnel.light.cloudy())
+        fresnel.geometry.Sphere(s, position=pos, radius=0.4, color=c,
+                                material=fresnel.material.Material(primitive_color_mix=1, roughness=0.5))
+        s.camera = fresnel.camera.Orthographic(position=(0, 0, 80), look_at=(0, 0, 0), up=(0, 1, 0), height=60)
+        return s
+
+    def image(t, s):
+        t.seed = 5
+        if tracer == 'Path':
+            t.sample(s, samples=1)
+        else:
+            t.render(s)
+        return numpy.array(t.linear_output[:])
+
+    def new_tracer():
+        return getattr(fresnel.tracer, tracer)(gpu_device, w=320, h=240)
+
+    fresh = [image(new_tracer(), build(c)) for c in colors]
+    assert not numpy.array_equal(*fresh)
+    s, t = build(colors[0]), new_tracer()
+    image(t, s)
+    builds = s._scene.bvhInfo()[0]
+    for k in range(8):
+        s.geometry[0].color[:] = colors[k % 2]
+        numpy.testing.assert_array_equal(image(t, s), fresh[k % 2])
+    assert s._scene.bvhInfo()[0] == builds
