@@ -677,6 +677,7 @@ struct SceneObj
     bool build_pending = false;  // a build or refit was queued on the device stream since its last sync
     DBuf<Node> nodes;
     DBuf<Node4> nodes4;
+    uint32_t types = 0;         // geometry types of the hierarchy as built (scene_types then)
     bool sphere_leaves = false; // leaf holds spheres (else bounds)
     DBuf<float4> leaf;          // leaf data in leaf order (SceneDev::leaf)
     DBuf<uint2> leaf_ref;
@@ -970,7 +971,8 @@ static void build_bvh(SceneObj& sc, bool refit_only)
         }
     sc.n_prims = N;
     sc.n_active = (uint32_t)slots.size();
-    sc.sphere_leaves = scene_types(sc) == T_SPHERES;
+    sc.types = scene_types(sc);
+    sc.sphere_leaves = sc.types == T_SPHERES;
     if (N == 0)
         {
         sc.bvh_valid = true;
@@ -1444,7 +1446,7 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
         const double xs = 0.5 * tr.W / tr.H + 2.0 / tr.H, ys = 0.5 + 2.0 / tr.H;
         c.plane_r = (float)(cam.focal_h * std::sqrt(xs * xs + ys * ys) * (1.0 + 0x1p-10));
         }
-    const bool spheres = scene_types(sc) == T_SPHERES;
+    const bool spheres = sc.sphere_leaves;
     const uint32_t n_tiles = c.tiles_x * c.tiles_y;
     // elements: primitives, or (other scenes, tile_group >= 2) the hierarchy
     // cut of kernels/tiles.hip over the N - 1 inner nodes; one more count
@@ -1453,7 +1455,7 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
     // for few lanes at a time, so polygon scenes take subtrees of at most 2
     // tiles (10,000 hexagons, 641 x 479, 64 samples: primary kernel 2.06 ms at
     // 4 tiles, 1.79 at 2; meshes 5.16 and 5.11, the mixed scene 7.1 and 7.4).
-    const uint32_t group = scene_types(sc) == (1u << G_POLYGON) ? std::min(D.tile_group, 2u) : D.tile_group;
+    const uint32_t group = sc.types == (1u << G_POLYGON) ? std::min(D.tile_group, 2u) : D.tile_group;
     const bool cut = !spheres && group >= 2 && N >= 2;
     const uint32_t n_inner = N - 1;
     const uint32_t n_el = cut ? 2 * n_inner + 2 : N + 1;
@@ -2320,7 +2322,7 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     // direct tracers do not support depth of field (fresnel/cpu/TracerDirect.cc:38-40)
     fh_user_camera cam = sc.camera;
     cam.f_stop = __builtin_huge_valf();
-    const bool own_search = (scene_types(sc) & (1u << G_POLYHEDRON)) != 0;
+    const bool own_search = (sc.types & (1u << G_POLYHEDRON)) != 0;
     if (!own_search)
         update_tiles(D, sc, tr, make_cam(cam), (uint64_t)tr.W * tr.H * tr.aa_n * tr.aa_n);
     JobDev J = make_job(sc, tr, cam);
@@ -2533,7 +2535,9 @@ static void server_plan(ServerObj& S)
         if (k[i] == 0)
             continue;
         RequestObj& r = S.reqs[ids[i]];
-        const uint32_t t = scene_types(*r.scene);
+        // as built: a geometry added, enabled or disabled since then shows once
+        // the scene is synchronized again, not in requests already admitted
+        const uint32_t t = r.scene->types;
         const int kd = (t & ~T_SPHERES) == 0 ? 0 : 1;
         // fewer samples (or none this step) when the batch would exceed its path limit
         const uint64_t pps = items[i].paths_per_sample;

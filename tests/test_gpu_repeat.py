@@ -3,7 +3,9 @@
 import numpy
 import pytest
 
+import bench
 import fresnel_amd as fresnel
+from fresnel_amd import serve
 from test_gpu_parity import c1_scene
 
 pytestmark = pytest.mark.gpu
@@ -105,3 +107,56 @@ def test_color_edits_reach_the_next_render(tracer, gpu_device):
         s.geometry[0].color[:] = colors[k % 2]
         numpy.testing.assert_array_equal(image(t, s), fresh[k % 2])
     assert s._scene.bvhInfo()[0] == builds
+
+
+@pytest.mark.parametrize('edit', ['add', 'enable', 'disable', 'disable_spheres'])
+def test_served_scene_edited_between_steps(edit, gpu_device):
+    """A geometry of another type added to, enabled or disabled in a served scene shows with the next synchronization:
+    the request goes on with the scene as it was built, and the next render has the edit."""
+
+    def build():
+        s = c1_scene(gpu_device, n=500)
+        if edit != 'add':
+            mesh(s)
+            if edit == 'enable':
+                s.geometry[1].disable()
+        return s
+
+    def mesh(s):
+        fresnel.geometry.Mesh(s, bench.icosphere(2.0, 1), position=[[0, 0, 9], [5, 5, 9]],
+                              orientation=[[1, 0, 0, 0]] * 2, color=(0.9, 0.2, 0.1))
+
+    def change(s):
+        if edit == 'add':
+            mesh(s)
+        elif edit == 'enable':
+            s.geometry[1].enable()
+        elif edit == 'disable':
+            s.geometry[1].disable()
+        else:
+            s.geometry[0].disable()
+
+    def sample(s):
+        t = fresnel.tracer.Path(gpu_device, w=72, h=56)
+        t.sample(s, samples=6)
+        return numpy.array(t.linear_output[:])
+
+    other = c1_scene(gpu_device, n=300, w_seed=3)
+    before, alone = sample(build()), sample(other)
+    edited = build()
+    change(edited)
+    after = sample(edited)
+    assert not numpy.array_equal(before, after)
+    s = build()
+    srv = serve.Server(gpu_device, hbm_budget=1 << 34, target_paths=2 * 72 * 56)
+    tracers = [fresnel.tracer.Path(gpu_device, w=72, h=56) for _ in range(2)]
+    reqs = [srv.submit(scene, t, 6) for scene, t in zip((s, other), tracers)]
+    for _ in range(2):
+        srv.step()  # both scenes are built
+    assert all(r.state == serve.ACTIVE for r in reqs)
+    change(s)
+    srv.run()
+    assert [r.state for r in reqs] == [serve.DONE] * 2
+    numpy.testing.assert_array_equal(tracers[0].linear_output[:], before)
+    numpy.testing.assert_array_equal(tracers[1].linear_output[:], alone)
+    numpy.testing.assert_array_equal(sample(s), after)
