@@ -297,6 +297,7 @@ struct DeviceObj
     std::vector<std::pair<std::string, std::pair<double, uint32_t>>> last_stats;
     uint64_t last_counters[N_CTR] = {};
     bool counters_zero = false; // the last render left every device counter zero, and nothing ran since
+    uint32_t server_batches = 0; // server batches started and not yet retired: they add to the counters
     std::mutex mu;
 
     hipEvent_t event()
@@ -376,7 +377,8 @@ struct DeviceObj
             std::memcpy(c, ctr, sizeof(c));
         else
             HIPCHECK(hipMemcpy(c, counters.p, sizeof(c), hipMemcpyDeviceToHost));
-        counters_zero = true;
+        // a server batch may have added to the counters after the copy
+        counters_zero = server_batches == 0;
         for (int k = 0; k < N_CTR; k++)
             {
             last_counters[k] = c[k];
@@ -2641,6 +2643,7 @@ static void server_finish_batch(ServerObj& S, size_t i)
     S.free_events.push_back(b.done);
     S.stage_pool.push_back(std::move(b.stage)); // its copies have completed
     S.batches.erase(S.batches.begin() + (std::ptrdiff_t)i);
+    D.server_batches--;
     if (q_flag)
         throw Error(FH_ERR_STATE, "internal error: a ray queue segment overflowed");
     if (s_flag)
@@ -2772,6 +2775,8 @@ static void server_step(ServerObj& S, double now, uint32_t& n_active, uint32_t& 
             }
         try
             {
+            D.server_batches++; // until server_finish_batch or the handler below
+            D.counters_zero = false;
             HIPCHECK(hipStreamWaitEvent(S.st[k], D.build_ev, 0));
             if (S.free_events.empty())
                 {
@@ -2795,7 +2800,6 @@ static void server_step(ServerObj& S, double now, uint32_t& n_active, uint32_t& 
                 }
             b.stage->ensure(stage_bytes(b.jobs.size()));
             b.e.reset(new BatchExec(D, S.rs[k], S.st[k], b.jobs, b.types, b.stage->p));
-            D.counters_zero = false;
             b.e->start();
             b.e->enqueue_kernels(D.steps_est);
             b.e->copy_counters();
@@ -2810,6 +2814,7 @@ static void server_step(ServerObj& S, double now, uint32_t& n_active, uint32_t& 
             {
             // whatever was enqueued drains; the batch's requests cannot complete
             (void)hipStreamSynchronize(S.st[k]);
+            D.server_batches--;
             for (auto& a : b.adds)
                 server_fail(S, a.first, now);
             S.batches.erase(S.batches.begin() + (std::ptrdiff_t)i);
@@ -3978,6 +3983,11 @@ extern "C"
                 for (int k = 0; k < 2; k++)
                     if (S.st[k])
                         (void)hipStreamSynchronize(S.st[k]);
+                {
+                std::lock_guard<std::mutex> lock(S.dev->mu);
+                for (auto& b : S.batches) // left by a drain that failed
+                    S.dev->server_batches -= b.stream >= 0 ? 1u : 0u;
+                }
                 for (hipEvent_t e : S.all_events)
                     (void)hipEventDestroy(e);
                 delete srv; // its streams are the device's

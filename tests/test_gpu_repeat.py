@@ -160,3 +160,41 @@ def test_served_scene_edited_between_steps(edit, gpu_device):
     numpy.testing.assert_array_equal(tracers[0].linear_output[:], before)
     numpy.testing.assert_array_equal(tracers[1].linear_output[:], alone)
     numpy.testing.assert_array_equal(sample(s), after)
+
+
+def test_counters_after_a_preview_beside_a_server_batch(gpu_device):
+    """A preview ends before a served batch has added its work to the device's counters: the next render still starts
+    from zero."""
+    d = gpu_device._device
+    alone = c1_scene(gpu_device, n=300)
+    t = fresnel.tracer.Path(gpu_device, w=64, h=48)
+
+    def counts():
+        t.seed = 7
+        t.sample(alone, samples=2)
+        return d.countersLast()
+
+    # few rays that take long: a polygon of 50,000 edges, 64 x 8 pixels
+    a = numpy.linspace(0, 2 * numpy.pi, 50000, endpoint=False)
+    slow = fresnel.Scene(gpu_device)
+    fresnel.geometry.Polygon(slow, numpy.stack([numpy.cos(a), numpy.sin(a)], axis=1), position=[[0, 0]])
+    slow.camera = fresnel.camera.Orthographic(position=(0, 0, 1), look_at=(0, 0, 0), up=(0, 1, 0), height=0.1)
+    small = fresnel.Scene(gpu_device)
+    fresnel.geometry.Sphere(small, position=[[0, 0, 0]], radius=0.5)
+    small.camera = fresnel.camera.Orthographic.fit(small)
+    preview = fresnel.tracer.Preview(gpu_device, w=8, h=8, anti_alias=False)
+    preview.render(small)
+    d.countersEnable(True)
+    try:
+        expected = counts()
+        srv = serve.Server(gpu_device, hbm_budget=1 << 34, target_paths=512)
+        req = srv.submit(slow, fresnel.tracer.Path(gpu_device, w=64, h=8), 8)
+        srv.step()
+        preview.render(small)
+        assert req.state == serve.ACTIVE
+        assert counts() == expected
+        srv.run()
+        assert req.state == serve.DONE
+        assert counts() == expected
+    finally:
+        d.countersEnable(False)
