@@ -381,6 +381,15 @@ __global__ void k_tile_cut(const Node* __restrict__ nodes, uint32_t n_inner, con
         }
     }
 
+// Whether a 32-bit exclusive scan of n counts ran over: an offset then lies
+// below the one before it (every count is below 2^32).
+__global__ void k_scan_wrapped(const uint32_t* __restrict__ offsets, uint32_t n, uint32_t* flags)
+    {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i + 1 < n && offsets[i + 1] < offsets[i])
+        atomicOr(flags, 2u);
+    }
+
 __global__ void k_gather_u32(const uint32_t* __restrict__ src, const uint32_t* __restrict__ idx, uint32_t n,
                              uint32_t* dst)
     {

@@ -1383,48 +1383,28 @@ struct TracerObj
         }
     };
 
-// Bring a tracer's per-tile candidate lists up to date for scene `sc` seen
-// through `cam` (pinhole perspective or orthographic cameras only; a scene a
-// perspective camera's plane cuts keeps the BVH search), for a render of
-// `n_pri` primary rays.  Building the lists costs about as much as the BVH
-// search loses on a few million primary rays, so they are built once the
-// primary rays rendered with one scene, camera and image size reach
-// D.tile_min_rays (this render's included); until then primary rays take the
-// BVH search.  Either way the hits are the same.
-static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev& cam, uint64_t n_pri)
+// Most entries a tracer's lists may have.  With the temporaries of their sorts
+// they take 60 bytes an entry, and k_tile_pack indexes two rows an entry with
+// 32 bits; a scene whose primitives each cover most of the image would have
+// them grow without bound.  Below that lists pay even there (10,000 spheres
+// over all of 1280 x 720 pixels, 1.4e8 entries: preview 43.8 ms by lists after
+// a first one of 69, 262 by packets; 16 path samples 37 and 90).
+constexpr uint32_t TILE_MAX_ENTRIES = 1u << 30;
+
+// Device memory of list builds back to the system (the device stream idle).
+static void release_tile_temps(TileTemps& X)
+    {
+    for (auto* b : {&X.counts, &X.tile0, &X.q0, &X.ref0, &X.keysA, &X.valsA, &X.keysB, &X.valsB, &X.hist})
+        b->release();
+    X.scan_tmp.clear();
+    }
+
+// Build the lists of tracer `tr` for scene `sc` seen through `cam`; tr.tiles
+// is valid afterwards unless the camera's plane cuts a primitive's box or the
+// lists would be too long.
+static void build_tile_lists(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev& cam)
     {
     TileLists& T = tr.tiles;
-    const bool pinhole = (cam.model == 1 && cam.a == 0.0f) || cam.model == 0;
-    if (D.primary_tiles != 2 || !pinhole || sc.n_prims == 0 || tr.W < TILE || tr.H < TILE)
-        {
-        T.valid = false;
-        T.decided = false;
-        T.scene = 0;
-        return;
-        }
-    if (T.scene == sc.serial && T.builds == sc.builds && T.refits == sc.refits && T.W == tr.W && T.H == tr.H
-        && T.group == D.tile_group && std::memcmp(&T.cam, &cam, sizeof(CamDev)) == 0)
-        {
-        if (T.decided)
-            return; // cached, usable or known unusable
-        T.rays += n_pri;
-        }
-    else
-        {
-        T.scene = sc.serial;
-        T.group = D.tile_group;
-        T.builds = sc.builds;
-        T.refits = sc.refits;
-        T.cam = cam;
-        T.W = tr.W;
-        T.H = tr.H;
-        T.valid = false;
-        T.decided = false;
-        T.rays = n_pri;
-        }
-    if (T.rays < D.tile_min_rays)
-        return;
-    T.decided = true;
     hipStream_t s = D.stream;
     const uint32_t N = sc.n_prims;
     TileCam c;
@@ -1480,13 +1460,17 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
                      k_tile_count<false><<<blocks(N + 1, 256), 256, 0, s>>>(sc.blo.p, sc.bhi.p, sc.dgeoms.p, N, c,
                                                                             X.counts.p, X.flags.p);
                  scan_exclusive(D, s, X.counts.p, n_el, X.scan_tmp);
+                 if ((uint64_t)(n_el - 1) * n_tiles >= 1ull << 32)
+                     k_scan_wrapped<<<blocks(n_el, 256), 256, 0, s>>>(X.counts.p, n_el, X.flags.p);
              });
     HIPCHECK(hipMemcpyAsync(&h[0], X.counts.p + (n_el - 1), 4, hipMemcpyDeviceToHost, s));
     HIPCHECK(hipMemcpyAsync(&h[1], X.flags.p, 4, hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     if (h[1])
-        return; // the camera plane cuts a primitive's box
+        return; // the camera plane cuts a primitive's box, or 2^32 entries and more
     const uint32_t M = h[0];
+    if (M > TILE_MAX_ENTRIES)
+        return;
     T.start.ensure(n_tiles);
     T.end.ensure(n_tiles);
     if (M > 0)
@@ -1547,6 +1531,63 @@ static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev
     T.tiles_y = c.tiles_y;
     T.n_entries = M;
     T.valid = true;
+    }
+
+// Bring a tracer's per-tile candidate lists up to date for scene `sc` seen
+// through `cam` (pinhole perspective or orthographic cameras only; a scene a
+// perspective camera's plane cuts, or whose lists would be too long, keeps the
+// BVH search), for a render of `n_pri` primary rays.  Building the lists costs
+// about as much as the BVH search loses on a few million primary rays, so they
+// are built once the primary rays rendered with one scene, camera and image
+// size reach D.tile_min_rays (this render's included); until then primary rays
+// take the BVH search.  Either way the hits are the same.
+static void update_tiles(DeviceObj& D, SceneObj& sc, TracerObj& tr, const CamDev& cam, uint64_t n_pri)
+    {
+    TileLists& T = tr.tiles;
+    const bool pinhole = (cam.model == 1 && cam.a == 0.0f) || cam.model == 0;
+    if (D.primary_tiles != 2 || !pinhole || sc.n_prims == 0 || tr.W < TILE || tr.H < TILE)
+        {
+        T.valid = false;
+        T.decided = false;
+        T.scene = 0;
+        return;
+        }
+    if (T.scene == sc.serial && T.builds == sc.builds && T.refits == sc.refits && T.W == tr.W && T.H == tr.H
+        && T.group == D.tile_group && std::memcmp(&T.cam, &cam, sizeof(CamDev)) == 0)
+        {
+        if (T.decided)
+            return; // cached, usable or known unusable
+        T.rays += n_pri;
+        }
+    else
+        {
+        T.scene = sc.serial;
+        T.group = D.tile_group;
+        T.builds = sc.builds;
+        T.refits = sc.refits;
+        T.cam = cam;
+        T.W = tr.W;
+        T.H = tr.H;
+        T.valid = false;
+        T.decided = false;
+        T.rays = n_pri;
+        }
+    if (T.rays < D.tile_min_rays)
+        return;
+    T.decided = true;
+    try
+        {
+        build_tile_lists(D, sc, tr, cam);
+        }
+    catch (const Error& e)
+        {
+        // no memory for lists: the BVH search needs none
+        if (e.code != FH_ERR_NOMEM)
+            throw;
+        (void)hipGetLastError();
+        HIPCHECK(hipStreamSynchronize(D.stream));
+        release_tile_temps(D.tile_tmp);
+        }
     }
 
 static JobDev make_job(SceneObj& sc, TracerObj& tr, const fh_user_camera& cam_user)

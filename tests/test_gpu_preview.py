@@ -54,3 +54,38 @@ def test_preview_lists_packets_checker(name, w, h, aa_n, gpu_device, cpu_device)
     ref = render(cpu_device, SCENES[name](cpu_device), w, h, aa_n)
     numpy.testing.assert_array_equal(lists[0][..., 3], ref[0][..., 3])
     numpy.testing.assert_allclose(lists[0], ref[0], rtol=4e-4, atol=1e-5)
+
+
+# 2^18 tiles, every sphere over all of them: lists of 2^27.8 entries; more than the 2^30 they may have; 2^32 + 3 * 2^18, whose
+# 32-bit count is 3 * 2^18
+@pytest.mark.parametrize('n,lists', [(900, True), (4100, False), (16387, False)])
+def test_preview_lists_too_long(n, lists, gpu_device):
+    """A scene whose lists would be too long is searched in the hierarchy: the same pixels as with lists off."""
+    d = gpu_device._device
+    s = fresnel.Scene(gpu_device, lights=fresnel.light.cloudy())
+    pos = numpy.random.default_rng(n).uniform(-1, 1, (n, 3))
+    fresnel.geometry.Sphere(s, position=pos, radius=5, color=(0.5, 0.5, 0.1))
+    s.camera = fresnel.camera.Orthographic(position=(0, 0, 30), look_at=(0, 0, 0), up=(0, 1, 0), height=2)
+    preview = fresnel.tracer.Preview(gpu_device, w=4096, h=4096, anti_alias=False)
+    path = fresnel.tracer.Path(gpu_device, w=4096, h=4096)
+
+    def images():
+        preview.render(s)
+        path.seed = 3
+        path.sample(s, samples=1)
+        return numpy.array(preview.output[:]), numpy.array(path.output[:])
+
+    d.statsEnable(True)
+    try:
+        preview.render(s)
+        assert ('tiles_emit' in d.statsLast()) == lists
+    finally:
+        d.statsEnable(False)
+    got = images()
+    try:
+        d.tune('primary_tiles', 1)
+        expected = images()
+    finally:
+        d.tune('primary_tiles', 2)
+    for a, b in zip(got, expected):
+        assert numpy.array_equal(a, b)
