@@ -2143,7 +2143,9 @@ static void update_live_frac(DeviceObj& D, const float* live)
 // order.  A batch's render stream waits, by event, for the work queued on the
 // device stream before it (scene builds, tile lists, output clears), so the
 // device stream can go on building the scenes of later batches meanwhile.
-// finish() returns with both render streams idle.
+// finish() returns with both render streams idle, and so does a run that an
+// error ends before: its batches use the pinned staging and the device's
+// render scratch, which the next call writes.
 struct InflightRun
     {
     DeviceObj& D;
@@ -2152,6 +2154,7 @@ struct InflightRun
     int slot = 0;
     size_t off = 0;
     uint32_t steps = 0;
+    bool finished = false;
     // the device counters after finish(): they only grow, so the largest of the
     // batches' copies
     unsigned long long ctr[N_CTR] = {};
@@ -2172,6 +2175,14 @@ struct InflightRun
             }
         D.stage.ensure(stage);
         steps = D.steps_est;
+        }
+    ~InflightRun()
+        {
+        if (!finished)
+            {
+            (void)hipStreamSynchronize(D.stream3);
+            (void)hipStreamSynchronize(D.stream2);
+            }
         }
 
     void add(std::vector<JobDev> jobs, uint32_t types)
@@ -2195,6 +2206,7 @@ struct InflightRun
         {
         HIPCHECK(hipStreamSynchronize(D.stream3));
         HIPCHECK(hipStreamSynchronize(D.stream2));
+        finished = true;
         uint32_t need = 0;
         float live[MAX_STEPS] = {};
         for (const auto& e : batches)

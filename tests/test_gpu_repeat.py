@@ -198,3 +198,30 @@ def test_counters_after_a_preview_beside_a_server_batch(gpu_device):
         assert counts() == expected
     finally:
         d.countersEnable(False)
+
+
+def test_preview_after_a_batch_that_failed(gpu_device):
+    """The second batch of a call is refused (2^32 light-sample paths) while the first one runs: the next call does not
+    touch what that one still uses."""
+    spheres = c1_scene(gpu_device, n=3000)
+    mesh = fresnel.Scene(gpu_device)
+    fresnel.geometry.Mesh(mesh, bench.icosphere(1.0, 1), position=[[0, 0, 0]], orientation=[[1, 0, 0, 0]])
+    mesh.camera = fresnel.camera.Orthographic.fit(mesh)
+    preview = fresnel.tracer.Preview(gpu_device, w=80, h=60)
+    path = fresnel.tracer.Path(gpu_device, w=640, h=480)
+
+    def images():
+        preview.render(mesh)
+        path.seed = 3
+        path.sample(spheres, samples=1, light_samples=2)
+        return numpy.array(preview.linear_output[:]), numpy.array(path.linear_output[:])
+
+    expected = images()
+    refused = fresnel.tracer.Path(gpu_device, w=256, h=256)
+    refused._tracer.setLightSamples(65535)
+    for _ in range(3):
+        path._tracer.setLightSamples(64)
+        with pytest.raises(RuntimeError, match='batch too large'):
+            fresnel._gpu.batch_render([spheres._scene, mesh._scene], [path._tracer, refused._tracer], 1)
+        for a, b in zip(images(), expected):
+            numpy.testing.assert_array_equal(a, b)
