@@ -298,6 +298,7 @@ struct DeviceObj
     uint64_t last_counters[N_CTR] = {};
     bool counters_zero = false; // the last render left every device counter zero, and nothing ran since
     uint32_t server_batches = 0; // server batches started and not yet retired: they add to the counters
+    std::atomic<uint64_t> clears {0}; // output clears queued on `stream` so far
     std::mutex mu;
 
     hipEvent_t event()
@@ -1326,6 +1327,10 @@ struct TracerObj
     DBuf<float4> linear;
     DBuf<uchar4> srgb;
     DBuf<uint32_t> hist; // histogram counts (512 x 4)
+    // a clear of the outputs was queued on the device stream, and nothing the
+    // host has waited for came after it; its number among the device's clears
+    bool clear_queued = false;
+    uint64_t clear_no = 0;
     std::vector<float> h_linear;
     std::vector<uint8_t> h_srgb;
     // asynchronous readback (fh_tracer_output_async): a pinned copy of each
@@ -1378,8 +1383,10 @@ struct TracerObj
         finish_copies();
         HIPCHECK(hipMemsetAsync(linear.p, 0, (size_t)W * H * sizeof(float4), dev->stream));
         HIPCHECK(hipMemsetAsync(srgb.p, 0, (size_t)W * H * sizeof(uchar4), dev->stream));
-        // not waited for: whatever reads or writes the outputs waits for the
-        // device stream (renders by event)
+        // not waited for: whatever writes the outputs waits for the device
+        // stream (renders by event), and so does a read before the next render
+        clear_no = ++dev->clears;
+        clear_queued = true;
         }
     };
 
@@ -2362,6 +2369,8 @@ static void render_path(DeviceObj& D, const std::vector<SceneObj*>& scenes, cons
     for (auto* tr : tracers)
         tr->n_samples += samples;
     D.end_stats(ctr);
+    for (auto* tr : tracers)
+        tr->clear_queued = false;
     if (D.last_counters[CTR_OVERFLOW])
         throw Error(FH_ERR_STATE, "traversal stack overflow");
     }
@@ -2407,6 +2416,7 @@ static void render_preview(DeviceObj& D, SceneObj& sc, TracerObj& tr)
     HIPCHECK(hipMemcpyAsync(ctr, D.counters.p, N_CTR * sizeof(*ctr), hipMemcpyDeviceToHost, D.stream));
     HIPCHECK(hipStreamSynchronize(D.stream));
     D.end_stats(ctr);
+    tr.clear_queued = false;
     if (D.last_counters[CTR_OVERFLOW])
         throw Error(FH_ERR_STATE, "traversal stack overflow");
     }
@@ -2458,6 +2468,7 @@ struct ServerBatch
     uint32_t types = 0;
     std::vector<std::pair<uint64_t, uint32_t>> adds; // (request, samples)
     uint64_t serial = 0;
+    uint64_t clears = 0; // output clears the batch waits for (DeviceObj::clears)
     int kind() const
         {
         return types == T_SPHERES ? 0 : 1;
@@ -2689,7 +2700,12 @@ static void server_finish_batch(ServerObj& S, size_t i)
         }
     const unsigned long long q_flag = b.e->h_ctr[CTR_QUEUE_OVERFLOW], s_flag = b.e->h_ctr[CTR_OVERFLOW];
     for (auto& a : b.adds)
-        S.reqs[a.first].done += a.second;
+        {
+        RequestObj& r = S.reqs[a.first];
+        r.done += a.second;
+        if (r.state == REQ_ACTIVE && r.tracer->clear_no <= b.clears)
+            r.tracer->clear_queued = false; // done before the batch began
+        }
     const int kd = b.kind();
     if (S.last_acc_batch[kd] == b.serial)
         S.last_acc[kd] = nullptr; // finished: later batches of its kind need not wait
@@ -2811,6 +2827,7 @@ static void server_step(ServerObj& S, double now, uint32_t& n_active, uint32_t& 
         if (b.stream >= 0)
             queued[b.stream]++;
     bool synced = false, started = false;
+    const uint64_t clears = D.clears;
     for (size_t i = 0; i < S.batches.size(); i++)
         {
         ServerBatch& b = S.batches[i];
@@ -2828,6 +2845,7 @@ static void server_step(ServerObj& S, double now, uint32_t& n_active, uint32_t& 
             }
         try
             {
+            b.clears = clears;
             D.server_batches++; // until server_finish_batch or the handler below
             D.counters_zero = false;
             HIPCHECK(hipStreamWaitEvent(S.st[k], D.build_ev, 0));
@@ -3748,7 +3766,11 @@ extern "C"
                 NONNULL(data);
                 TracerObj& T = tr->obj;
                 const size_t n = (size_t)T.W * T.H;
-                HIPCHECK(hipStreamSynchronize(T.dev->stream)); // a clear may still be queued
+                // the device stream may hold other requests' scene builds: it is
+                // waited for only if the outputs' clear may still be queued there
+                if (T.clear_queued)
+                    HIPCHECK(hipStreamSynchronize(T.dev->stream));
+                T.clear_queued = false;
                 if (which == FH_OUT_SRGB)
                     {
                     HIPCHECK(hipMemcpy(T.h_srgb.data(), T.srgb.p, n * 4, hipMemcpyDeviceToHost));

@@ -1,5 +1,7 @@
 """Repeated renders of one scene and tracer: what a call leaves out must not show."""
 
+import time
+
 import numpy
 import pytest
 
@@ -225,3 +227,40 @@ def test_preview_after_a_batch_that_failed(gpu_device):
             fresnel._gpu.batch_render([spheres._scene, mesh._scene], [path._tracer, refused._tracer], 1)
         for a, b in zip(images(), expected):
             numpy.testing.assert_array_equal(a, b)
+
+
+def test_reading_an_image_does_not_wait_for_other_work(gpu_device):
+    """A finished image (of Path.sample or a server) is read at once while clears of other outputs (33 GB) are still
+    queued on the device stream; those outputs are read only after theirs."""
+    s = c1_scene(gpu_device, n=300)
+    sampled, served = [fresnel.tracer.Path(gpu_device, w=64, h=48) for _ in range(2)]
+    preview = fresnel.tracer.Preview(gpu_device, w=64, h=48)
+    sampled.sample(s, samples=2)
+    preview.render(s)
+    srv = serve.Server(gpu_device, hbm_budget=1 << 34, target_paths=1 << 16)
+    req = srv.submit(s, served, 2)
+    srv.run()
+    assert req.state == serve.DONE
+    images = [numpy.array(t.linear_output[:]) for t in (sampled, served, preview)]
+    large = fresnel.tracer.Path(gpu_device, w=4096, h=4096)
+    large.output[:]
+
+    def timed(read):
+        times = []
+        for _ in range(3):
+            for _ in range(100):
+                large.reset()
+            t0 = time.perf_counter()
+            read()
+            times.append(time.perf_counter() - t0)
+            large.histogram()  # waits for the device stream
+        return min(times)
+
+    wait = timed(large.histogram)
+    for t, image in zip((sampled, served, preview), images):
+        assert timed(lambda: t.linear_output[:]) < 0.5 * wait
+        numpy.testing.assert_array_equal(t.linear_output[:], image)
+    large.sample(s, samples=1)
+    for _ in range(20):
+        large.reset()
+    assert not large.output[:].any()
