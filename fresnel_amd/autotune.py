@@ -23,7 +23,8 @@ for every setting; only speed changes.  Knobs (see fh_device_tune):
                   used one scene and camera.
 * ``tile_group`` largest tile count of a hierarchy subtree listed as one
                   tile-list entry (scenes other than spheres-only; 1: one
-                  entry per primitive).
+                  entry per primitive; the default 4 counts as 2 in scenes of
+                  polygons only).
 * ``fuse_primary`` primary traversal and depth-0 shading in one kernel (2) or
                   two (1).
 * ``fuse_bounce`` the same for each bounce of the secondary rays.

@@ -208,6 +208,9 @@ struct PinnedBuf
         }
     };
 
+// Default of DeviceObj::tile_group (polygon scenes take 2 tiles for it, build_tile_lists).
+constexpr uint32_t TILE_GROUP = 4;
+
 // Bounce steps a batch can be given: the last one finishes every path left.
 constexpr uint32_t MAX_STEPS = 64;
 
@@ -271,7 +274,7 @@ struct DeviceObj
     uint32_t primary_chunk = 1024;      // the most primary rays a workgroup claims at once
     uint32_t trav_packet = 2;           // primary rays: 2 wavefront packets, 1 per ray
     uint32_t primary_tiles = 2;         // primary rays of pinhole/orthographic cameras: 2 tile lists, 1 BVH
-    uint32_t tile_group = 4;            // tile-list subtrees cover at most this many tiles (1: primitives only)
+    uint32_t tile_group = TILE_GROUP;   // tile-list subtrees cover at most this many tiles (1: primitives only)
     uint64_t tile_min_rays = 4ull << 20; // tile lists once this many primary rays used one scene and camera
     uint32_t fuse_primary = 2;          // 2: primary traversal and depth-0 shading in one kernel, 1: two
     uint32_t fuse_bounce = 1;           // 2: secondary traversal and shading in one kernel, 1: two
@@ -1440,11 +1443,15 @@ static void build_tile_lists(DeviceObj& D, SceneObj& sc, TracerObj& tr, const Ca
     // elements: primitives, or (other scenes, tile_group >= 2) the hierarchy
     // cut of kernels/tiles.hip over the N - 1 inner nodes; one more count
     // slot holds the scan's total
-    // A polygon's test is the longest (every edge), and a subtree entry runs it
-    // for few lanes at a time, so polygon scenes take subtrees of at most 2
-    // tiles (10,000 hexagons, 641 x 479, 64 samples: primary kernel 2.06 ms at
-    // 4 tiles, 1.79 at 2; meshes 5.16 and 5.11, the mixed scene 7.1 and 7.4).
-    const uint32_t group = sc.types == (1u << G_POLYGON) ? std::min(D.tile_group, 2u) : D.tile_group;
+    // By default polygon scenes take subtrees of 2 tiles, whatever the number
+    // of edges: their boxes lie in one plane, so no entry ends a list early and
+    // a subtree searched by few lanes at a time is only serial work (primary
+    // kernel at 2 and 4 tiles, 641 x 479, 64 samples: 10,000 triangles 1.25
+    // and 1.55 ms, hexagons 1.49 and 1.86, of 64 edges 6.8 and 7.4; 100,000
+    // triangles 4.5 and 5.5, hexagons 5.7 and 6.8; 1,000 of each the same.
+    // Meshes 5.11 and 5.16, the mixed scene 7.4 and 7.1).  Another tile_group
+    // than the default is taken as given.
+    const uint32_t group = (sc.types == (1u << G_POLYGON) && D.tile_group == TILE_GROUP) ? 2u : D.tile_group;
     const bool cut = !spheres && group >= 2 && N >= 2;
     const uint32_t n_inner = N - 1;
     const uint32_t n_el = cut ? 2 * n_inner + 2 : N + 1;

@@ -334,7 +334,8 @@ int fh_policy_simulate(uint32_t n, const uint64_t* footprint, const uint64_t* pa
  * scenes other than spheres-only, those lists hold hierarchy subtrees whose
  * tile rectangle covers at most this many tiles (a mesh instance's triangles
  * become one entry, searched only by the rays that pass its box), 2..1024, or
- * 1 for one entry per primitive (default 4); "fuse_primary":
+ * 1 for one entry per primitive (default 4, which scenes of polygons only
+ * take as 2); "fuse_primary":
  * primary traversal and depth-0 shading in one kernel (2, default) or two (1);
  * "fuse_bounce": the same for each bounce of the secondary rays (default 1:
  * the fused kernel holds 88 registers, and the latency-bound secondary

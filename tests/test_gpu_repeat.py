@@ -264,3 +264,33 @@ def test_reading_an_image_does_not_wait_for_other_work(gpu_device):
     for _ in range(20):
         large.reset()
     assert not large.output[:].any()
+
+
+def test_tile_group_of_polygon_scenes(gpu_device):
+    """Polygon scenes take the default tile_group as 2 tiles and every other value as it is: the entries tested differ,
+    the images do not."""
+    rng = numpy.random.default_rng(2)
+    s = fresnel.Scene(gpu_device, lights=fresnel.light.cloudy())
+    fresnel.geometry.Polygon(s, [[-0.1, -0.1], [0.1, -0.1], [0, 0.1]], position=rng.uniform(-5, 5, (4000, 2)),
+                             angle=rng.uniform(0, 6, 4000), color=(0.2, 0.5, 0.9))
+    s.camera = fresnel.camera.Orthographic(position=(0, 0, 5), look_at=(0, 0, 0), up=(0, 1, 0), height=10)
+    t = fresnel.tracer.Path(gpu_device, w=203, h=151)
+    d = gpu_device._device
+    default = d.tune('tile_group', 0)
+    assert default == 4
+    entries, images = {}, {}
+    d.countersEnable(True)
+    try:
+        for group in (1, 2, 4, 9, 16):
+            d.tune('tile_group', group)
+            t.seed = 3
+            t.sample(s, samples=2)
+            entries[group] = d.countersLast()[10]
+            images[group] = numpy.array(t.linear_output[:])
+    finally:
+        d.countersEnable(False)
+        d.tune('tile_group', default)
+    assert entries[4] == entries[2]
+    assert len({entries[g] for g in (1, 2, 9, 16)}) == 4
+    for group in images:
+        numpy.testing.assert_array_equal(images[group], images[1])
