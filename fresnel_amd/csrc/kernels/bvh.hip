@@ -523,8 +523,11 @@ __device__ __forceinline__ void child_box(const Node& n, uint32_t side, float b[
 // On each axis the children's boxes are rounded outwards to 8-bit steps of
 // the node's own interval, after a pad of 2^-20 of the node's largest
 // coordinate: what the search's slab test loses to rounding (search_visit).
-// An infinite or NaN end becomes one beyond every finite scene; a primitive's
-// own bounds are tested exactly at its leaf.
+// An end that is infinite, NaN or beyond 2^66 becomes -2^66 (a low end) or 2^66
+// (a high one), the largest interval whose slab test cannot overflow (2^67
+// times RCP_MAX, 2^60), above the 2^64 at which squared distances overflow in
+// the primitives' own tests.  A primitive's own bounds are tested exactly at
+// its leaf, so one out there is still found by every ray that starts within.
 __global__ void k_bvh4_fill(const Node* __restrict__ nodes, uint32_t n, const uint32_t* __restrict__ idx4,
                             const uint32_t* __restrict__ parent, Node4* __restrict__ out)
     {
@@ -579,7 +582,7 @@ __global__ void k_bvh4_fill(const Node* __restrict__ nodes, uint32_t n, const ui
         ref[1] = ref[0];
         m = 2;
         }
-    constexpr float FAR = 1e18f;
+    constexpr float FAR = 0x1p66f;
     float big = 0.0f;
     for (uint32_t k = 0; k < m; k++)
         for (int x = 0; x < 6; x++)

@@ -43,6 +43,7 @@ SCENES = {
     'spheres_700': spheres(700, 8.0, radius=0.02),
     'spheres_milli': spheres(200, 1e-3),
     'spheres_mega': spheres(200, 1e6),
+    'spheres_1e18': spheres(200, 1e18),
     'spheres_aside': spheres(200, 1.0, offset=1000.0),
     'c1': c1_scene,
     'flat': flat,
