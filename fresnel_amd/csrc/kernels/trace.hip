@@ -139,7 +139,7 @@ template<int SS> struct LdsStack
         }
     };
 
-// Stack in private memory (for the preview and diagnostic kernels).
+// Stack in private memory (for the diagnostic kernels).
 struct LocalStack
     {
     uint2 s[STACK_MAX];

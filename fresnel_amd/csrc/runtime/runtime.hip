@@ -244,6 +244,7 @@ struct DeviceObj
     std::string name;
     int limit = -1;
     uint32_t trav_grid = 0;
+    uint32_t finish_grid = 0; // largest resident grid of any tail kernel variant
     RenderScratch rs, rs2; // render scratch of the two batches in flight
     PinnedBuf stage;       // job tables, pixel bases and step records of one render's batches
     uint32_t graph = 1;     // 2: a batch's kernels are captured once into a HIP graph and replayed; 1: launched
@@ -593,6 +594,25 @@ template<int SS> static uint32_t max_grid_ss(DeviceObj& D)
                           reinterpret_cast<const void*>(&k_bounce<TRAV_BLOCK, SS, true, T_ALL>)})
         g = std::max(g, D.grid_for(k, TRAV_BLOCK));
     return g;
+    }
+
+// Largest resident grid of any tail kernel variant (sizes its overflow stacks).
+static uint32_t max_finish_grid(DeviceObj& D)
+    {
+    uint32_t g = 0;
+    for (const void* k : {reinterpret_cast<const void*>(&k_finish<TRAV_BLOCK, TRAV_SS, false, T_SPHERES>),
+                          reinterpret_cast<const void*>(&k_finish<TRAV_BLOCK, TRAV_SS, true, T_SPHERES>),
+                          reinterpret_cast<const void*>(&k_finish<TRAV_BLOCK, TRAV_SS, false, T_ALL>),
+                          reinterpret_cast<const void*>(&k_finish<TRAV_BLOCK, TRAV_SS, true, T_ALL>)})
+        g = std::max(g, D.grid_for(k, TRAV_BLOCK));
+    return g;
+    }
+
+// Entries of the tail kernel's overflow stacks: its resident threads, or one a
+// path when fewer paths may reach it.
+static size_t tail_stack_entries(const DeviceObj& D)
+    {
+    return (size_t)(STACK_MAX - TRAV_SS) * std::min(D.finish_grid, blocks(D.tail_rays, TRAV_BLOCK)) * TRAV_BLOCK;
     }
 
 // ====================================================================== geometry
@@ -1718,7 +1738,7 @@ struct BatchExec
     uint32_t types;
     bool spheres;
     uint64_t n_pri = 0, n_paths = 0, n_pix = 0, n_rec = 0;
-    uint32_t nj = 0, gstride = 0, seg_cap = 0, tail_threads = 0, rest_grid = 0, tail_grid = 0;
+    uint32_t nj = 0, gstride = 0, seg_cap = 0, rest_grid = 0, tail_grid = 0;
     uint32_t pgroups = 1; // primary claim size in workgroups of rays (primary_groups)
     uint32_t n_steps = 0;
     int cur = 1;
@@ -1775,11 +1795,10 @@ struct BatchExec
         // growing a buffer frees it first: an earlier batch on this stream
         // (the only user of this scratch) must have finished with it
         gstride = D.trav_grid * TRAV_BLOCK; // max resident threads of any traversal variant
-        tail_threads = blocks(D.tail_rays, TRAV_BLOCK) * TRAV_BLOCK;
         const bool fits = R.hits.cap >= std::max(n_pri, n_paths) && R.qo[0].cap >= cap && R.qo[1].cap >= cap
                           && R.records.cap >= n_rec && R.jobs.cap >= jobs.size()
                           && R.gstack.cap >= (size_t)(STACK_MAX - 8) * gstride
-                          && R.tail_stack.cap >= (size_t)(STACK_MAX - TRAV_SS) * tail_threads && R.view.p && R.counters32.p && R.qseg.p;
+                          && R.tail_stack.cap >= tail_stack_entries(D) && R.view.p && R.counters32.p && R.qseg.p;
         if (!fits)
             HIPCHECK(hipStreamSynchronize(s));
         R.hits.ensure(std::max(n_pri, n_paths));
@@ -1806,8 +1825,7 @@ struct BatchExec
         p += (2 * MAX_STEPS * sizeof(uint32_t) + 255) & ~(size_t)255;
         h_ctr = (unsigned long long*)p;
         R.gstack.ensure((size_t)(STACK_MAX - 8) * gstride);
-        // the tail kernel's grid-stride threads (at least tail_rays)
-        R.tail_stack.ensure((size_t)(STACK_MAX - TRAV_SS) * tail_threads);
+        R.tail_stack.ensure(tail_stack_entries(D));
         for (int q = 0; q < 2; q++)
             {
             Q[q] = Queue {R.qo[q].p, R.qd[q].p, R.qatt[q].p, R.qmeta[q].p};
@@ -1822,7 +1840,7 @@ struct BatchExec
                                SHADE_BLOCK);
         // resident grid of the tail kernel, within its overflow stacks
         tail_grid = std::min(D.grid_for(reinterpret_cast<const void*>(finish_kernel()), TRAV_BLOCK),
-                             tail_threads / TRAV_BLOCK);
+                             blocks(D.tail_rays, TRAV_BLOCK));
         }
 
     auto finish_kernel() const -> decltype(&k_finish<TRAV_BLOCK, TRAV_SS, false, T_ALL>)
@@ -1853,7 +1871,7 @@ struct BatchExec
     std::vector<uint64_t> graph_key(uint32_t steps) const
         {
         std::vector<uint64_t> k = {(uint64_t)(uintptr_t)s, nj, n_pri, n_paths, n_pix, n_rec, seg_cap, gstride,
-                                   tail_threads, types, steps, D.trav_chunk, pgroups, D.xcd_bands,
+                                   types, steps, D.trav_chunk, pgroups, D.xcd_bands,
                                    D.fuse_primary, D.fuse_bounce, D.tail_rays, (uint64_t)D.stack_lds, D.trav_refill,
                                    D.trav_packet, D.count_on ? 1u : 0u, rest_grid, tail_grid,
                                    per_ray_primary() ? 1u : 0u};
@@ -2527,8 +2545,7 @@ static uint64_t server_reserved(const ServerObj& S)
     {
     const DeviceObj& D = *S.dev;
     const uint64_t fixed = (uint64_t)(STACK_MAX - 8) * D.trav_grid * TRAV_BLOCK * sizeof(uint2)
-                           + (uint64_t)(STACK_MAX - TRAV_SS) * blocks(D.tail_rays, TRAV_BLOCK) * TRAV_BLOCK
-                                 * sizeof(uint2);
+                           + tail_stack_entries(D) * sizeof(uint2);
     uint64_t device_scratch = 0;
     for (const RenderScratch* R : {&D.rs, &D.rs2})
         {
@@ -3054,6 +3071,7 @@ extern "C"
                     HIPCHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
                 // overflow stacks are sized for the largest resident traversal grid
                 D.trav_grid = std::max(max_grid_ss<8>(D), max_grid_ss<16>(D));
+                D.finish_grid = max_finish_grid(D);
                 if (const char* e = getenv("FRESNEL_AMD_BATCH_PATHS"))
                     D.batch_paths = std::max<uint64_t>(1, strtoull(e, nullptr, 10));
                 if (const char* e = getenv("FRESNEL_AMD_TAIL_RAYS"))

@@ -294,3 +294,22 @@ def test_tile_group_of_polygon_scenes(gpu_device):
     assert len({entries[g] for g in (1, 2, 9, 16)}) == 4
     for group in images:
         numpy.testing.assert_array_equal(images[group], images[1])
+
+
+def test_tail_threshold_takes_no_memory(gpu_device):
+    """The tail kernel's overflow stacks belong to its resident threads: a threshold of 2^24 rays keeps no request out
+    of an 8 GB budget (a stack for each ray would take 10.7 GB in each of two scratches)."""
+    s = c1_scene(gpu_device, n=3000)
+    alone = fresnel.tracer.Path(gpu_device, w=96, h=64)
+    alone.sample(s, samples=3)
+    d = gpu_device._device
+    old = d.tune('tail_rays', 1 << 24)
+    try:
+        srv = serve.Server(gpu_device, hbm_budget=8 << 30, target_paths=1 << 20)
+        t = fresnel.tracer.Path(gpu_device, w=96, h=64)
+        req = srv.submit(s, t, 3)
+        srv.run()
+        assert req.state == serve.DONE
+        numpy.testing.assert_array_equal(t.linear_output[:], alone.linear_output[:])
+    finally:
+        d.tune('tail_rays', old)
