@@ -41,7 +41,8 @@ __device__ __forceinline__ void slab(v3 o, v3 inv, float lx, float ly, float lz,
 // slab interval is [tmin, tmax] (see CULL_K).  A box is culled when this
 // bound exceeds the closest hit, so every primitive that could still win is
 // tested and the result does not depend on the hierarchy or the visiting
-// order.  margin = CULL_K * 3 * the scene's largest primitive half-extent.
+// order (but for polyhedra's hits below their bound, CULL_K).  margin = CULL_K
+// * 3 * the scene's largest primitive half-extent.
 __device__ __forceinline__ float cull_bound(float tmin, float tmax, float margin)
     {
     return tmin - (CULL_K * fmaxf(tmax, 0.0f) + margin);
@@ -433,9 +434,12 @@ __device__ inline void trace_binary(const SceneDev& sc, v3 o, v3 d, float tnear,
 // A child is culled when its key, max(tmin, 0) - CULL_K tmax, exceeds the
 // closest hit plus the scene's margin (cull_bound with the margin moved to
 // the other side; CULL_K's factor of two covers the roundings of key and sum).
-// So every primitive whose bounds pass the slab test and that could still win
-// is tested, and the result is the smallest (t, geometry, primitive) whatever
-// the hierarchy and the order.
+// So every primitive whose bounds pass the slab test and whose hit does not lie
+// below its own culling bound is tested if it could still win, and the result
+// is the smallest (t, geometry, primitive) of those whatever the hierarchy and
+// the order.  Only polyhedra have hits below that bound (CULL_K): where one is
+// the smallest, this search and the binary one may differ, as either may from
+// the checker's.
 //
 // Bound by VALU issue (99 % on the lattice) with under half the lanes active.
 // Exact boxes and leaf tests on the spot took about 450 instructions per
@@ -2453,9 +2457,9 @@ __device__ __forceinline__ float4 preview_shade(const JobDev& J, const HitT& h, 
 // order of the reference's loop, so the sum does not depend on the split).
 // Otherwise (fewer samples than wavefronts) each wavefront has a chunk to
 // itself.  own_search: each lane searches the binary hierarchy for its own ray
-// (scenes with convex polyhedra: a face nearly parallel to a ray gives a
-// computed distance up to units below its box's entry, so which hit is found
-// first decides, and the order stays that of the search per ray).
+// (scenes with convex polyhedra, whose hits may lie units below their box's
+// entry, see CULL_K: which one is found first decides then, and the order stays
+// that of the search per ray).
 // The kernel is bound by VALU issue (camera rays with Philox, the
 // lights' acos, sin and cos).  One pixel per thread with its own search and
 // 64 serial samples, in raster order with the stack in scratch, took 5.99 ms

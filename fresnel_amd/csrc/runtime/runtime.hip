@@ -1901,8 +1901,8 @@ struct BatchExec
     // spherocylinders at 3.9, 16 and 63 0.26 / 0.38, 0.44 / 0.46, 0.70 / 0.56,
     // triangles at 13, 50 and 200 0.33 / 0.37, 0.47 / 0.45, 0.86 / 0.58.
     // Spheres stay with packets (their test is the cheapest: 1.56 / 1.62 at
-    // 78), as do tile lists, and scenes with polyhedra, whose grazing faces
-    // make a hit depend on the search's order (k_preview).
+    // 78), as do tile lists, and scenes with polyhedra, whose hits below their
+    // bound (CULL_K) depend on the search's order.
     bool per_ray_primary() const
         {
         if (spheres || (types & (1u << G_POLYHEDRON)) || D.fuse_primary != 2 || D.trav_packet != 2)

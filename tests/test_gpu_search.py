@@ -90,3 +90,61 @@ def test_search_equals_brute_force(name, tnear, gpu_device, cpu_device):
     assert numpy.array_equal(prim, rp)
     assert numpy.array_equal(t.view(numpy.uint32), rt.view(numpy.uint32))
     assert (rg != 0xffffffff).any()
+
+
+CUBOID = [[x, y, z] for x in (-0.5, 0.5) for y in (-0.5, 0.5) for z in (-0.25, 0.25)]
+
+
+def test_edge_lines_of_polyhedra(gpu_device, cpu_device):
+    """Rays through the lines of edges beyond the edges' ends, in a dense scene of convex polyhedra.  The reference's plane
+    loop ends when the largest entry and smallest exit distance are equal and reports a hit, the planes left unseen, so
+    such a ray, though it passes outside, may hit a polyhedron far before its bounding box.  The search then may or may not
+    meet that hit before a nearer one culls its box.  Every other hit is the brute-force minimum: a ray that differs from
+    brute force has a brute-force hit below that primitive's own culling bound."""
+    n, n_rays, side = 3000, 200000, 20.0
+    rng = numpy.random.default_rng(8)
+    pos = rng.uniform(-side / 2, side / 2, (n, 3)).astype(numpy.float32)
+    q = rng.normal(size=(n, 4))
+    q = (q / numpy.linalg.norm(q, axis=1, keepdims=True)).astype(numpy.float32)
+
+    def build(device):
+        s = fresnel.Scene(device)
+        fresnel.geometry.ConvexPolyhedron(s, fresnel.util.convex_polyhedron_from_vertices(CUBOID), position=pos,
+                                          orientation=q)
+        return s
+
+    # a point on the line of an edge of polyhedron k, past the edge's end; rays through it from 20 to 130 away
+    half, radius = numpy.array(CUBOID[-1]), numpy.linalg.norm(CUBOID[-1])
+    k = rng.integers(0, n, n_rays)
+    p = half * rng.choice([-1, 1], (n_rays, 3))
+    axis = rng.integers(0, 3, n_rays)
+    p[numpy.arange(n_rays), axis] *= rng.uniform(1, radius / half[axis])
+    d = rng.normal(size=(n_rays, 3))
+    d /= numpy.linalg.norm(d, axis=1, keepdims=True)
+
+    def rotate(x):
+        s, v = q[k].astype(numpy.float64)[:, :1], q[k].astype(numpy.float64)[:, 1:]
+        return x + 2 * numpy.cross(v, numpy.cross(v, x) + s * x)
+
+    o = p - d * rng.uniform(20, 130, (n_rays, 1))
+    rays = numpy.ascontiguousarray(numpy.concatenate([rotate(o) + pos[k], rotate(d)], axis=1), dtype=numpy.float32)
+    gs, cs = build(gpu_device), build(cpu_device)
+    gid, prim, t = gs._scene.debugTrace(rays, 1e-3)
+    L, h = oracle.lib(), cs._scene.handle()
+    L.oracle_scene_set_brute(h, 1)
+    rg, rp, rt = (numpy.zeros(n_rays, numpy.uint32), numpy.zeros(n_rays, numpy.uint32),
+                  numpy.zeros(n_rays, numpy.float32))
+    L.oracle_trace(h, ptr(rays), n_rays, 1e-3, ptr(rg, ctypes.c_uint32), ptr(rp, ctypes.c_uint32), ptr(rt), None, 0)
+    hit = rg != 0xffffffff
+    # the culling bound of the brute-force winner: its box's slab interval, less 2^-9 of its end and of 3 half extents
+    with numpy.errstate(divide='ignore'):
+        inv = 1 / rays[:, 3:].astype(numpy.float64)
+    a = (pos[rp * hit] - radius - rays[:, :3]) * inv
+    b = (pos[rp * hit] + radius - rays[:, :3]) * inv
+    tmin, tmax = numpy.minimum(a, b).max(axis=1), numpy.maximum(a, b).min(axis=1)
+    bound = tmin - 2.0**-9 * (numpy.maximum(tmax, 0) + 3 * radius)
+    below = hit & (rt < bound * (1 + 1e-5))
+    differs = (gid != rg) | (prim != rp) | (t.view(numpy.uint32) != rt.view(numpy.uint32))
+    print(f"{below.sum()} of {hit.sum()} hits below their own bound, {differs.sum()} rays differ from brute force")
+    assert below.any()
+    assert not (differs & ~below).any()
