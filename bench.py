@@ -15,8 +15,9 @@ the timed region).  Mpaths/s = W*H*samples*light_samples per second.  The
 JSON line also carries:
   roofline         the kernel with the most time per frame (the
                    secondary-ray traversal or the fused primary kernel):
-                   algorithmic bytes per launch (64 B per hierarchy node visit,
-                   4-wide or binary, prim_bytes per primitive tested, the ray's own bytes, from
+                   algorithmic bytes per launch (64 B per hierarchy node
+                   visit, 4-wide or binary, prim_bytes per primitive tested,
+                   the ray's own bytes, from
                    the instrumented work counters) over the average launch
                    duration (HIP events on the stream it runs on), against
                    8 TB/s HBM; beside it the same launches' model FP32 flops
@@ -481,8 +482,8 @@ def run_plain(args):
     seg_rays = ctr[0] + ctr[3] + ctr[6]
     path_bytes = (node_bytes * (ctr[1] + ctr[4] + ctr[7]) + pb * (ctr[2] + ctr[5] + ctr[8])
                   + 36 * W * H * S)
-    path_flops = (FLOPS_PER_NODE4 * (ctr[1] + ctr[7]) + FLOPS_PER_NODE2 * ctr[4] + FLOPS_PER_SPHERE * (ctr[2] + ctr[5] + ctr[8])
-                  + FLOPS_PER_RAY * seg_rays)
+    path_flops = (FLOPS_PER_NODE4 * (ctr[1] + ctr[7]) + FLOPS_PER_NODE2 * ctr[4]
+                  + FLOPS_PER_SPHERE * (ctr[2] + ctr[5] + ctr[8]) + FLOPS_PER_RAY * seg_rays)
     kernel_ms = {k: round(v[0], 3) for k, v in kstats[-1].items()}
     kernel_launches = {k: int(v[1]) for k, v in kstats[-1].items()}
 

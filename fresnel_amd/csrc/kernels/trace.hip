@@ -553,7 +553,11 @@ __device__ __forceinline__ void order2(float& ka, uint32_t& na, float& kb, uint3
     }
 
 // One node visit: the nearest open child is taken next, the others are pushed,
-// farthest first.
+// farthest first.  The near distance is held at 0, not at tnear, so a ray that
+// leaves a surface opens the padded boxes it starts in: in flat systems that
+// costs visits (polygons: 8.3 a secondary ray, the binary tree with its exact
+// boxes and tnear 1.0), with tnear in its place 10,000 hexagons took 4 % less
+// a call and 4,096 spheres 2 % more.
 template<class Stack, bool COUNT>
 __device__ __forceinline__ void search_visit(const Node4* __restrict__ nodes, Search& r, Stack& st, uint32_t& n_nodes,
                                              uint32_t& err)
@@ -660,8 +664,8 @@ __device__ __forceinline__ void test_type(const GeomDev* __restrict__ geoms, Sea
     }
 
 // Leaf step in other scenes (the leaf array's form depends on the scene:
-// kernels of other types are never given a spheres-only scene): the gate with the stored bounds, then one
-// geometry type at a time.
+// kernels of other types are never given a spheres-only scene): the gate with
+// the stored bounds, then one geometry type at a time.
 template<uint32_t TYPES, bool COUNT, bool UNI>
 __device__ __forceinline__ void search_mixed(const SearchScene<UNI>& sc, Search& r, uint32_t& n_prims)
     {
@@ -1168,7 +1172,8 @@ struct Claims
 // with 64 rays at a time to their ends, and so: lattice of 1M spheres 9.0 and
 // 8.3 ms, small scene 0.55 and 0.36, meshes 9.1 and 6.0, mixed 9.5 and 5.9,
 // spherocylinders 2.2 and 1.0 (refill at 16, 24, 32, 40 idle lanes: lattice
-// 8.8, 8.7, 8.4, 8.1, meshes 6.1, 6.0, 6.2, 6.3, mixed 5.95, 5.98, 6.01, 6.19).
+// 8.8, 8.7, 8.4, 8.1, meshes 6.1, 6.0, 6.2, 6.3, mixed 5.95, 5.98, 6.01, 6.19:
+// 32 serves both kernels, spheres alone would take 40).
 // Held to 7 wavefronts per SIMD in spheres-only scenes (6: lattice 8.8; 8
 // spills), 6 otherwise (5: mixed 6.4, 7: meshes 7.5 against 6.9 then).
 template<int BLOCK, int SS, bool COUNT, bool PRIMARY, uint32_t TYPES>
@@ -1956,8 +1961,8 @@ __global__ __launch_bounds__(BLOCK) void k_traverse_packet(const JobDev* __restr
                 primary_ray(jobs, n_jobs, i, job, k, px, py, jord, o, d);
                 }
             HitT best;
-            primary_group_hit<SS, COUNT, TYPES, false>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes, n_prims,
-                                                n_entries, err);
+            primary_group_hit<SS, COUNT, TYPES, false>(jobs, valid, job, px, py, o, d, 1e-3f, st, best, n_nodes,
+                                                       n_prims, n_entries, err);
             if (valid)
                 {
                 hits[i] = make_uint4(__float_as_uint(best.t), best.geom, best.prim, 0);
@@ -2470,9 +2475,9 @@ __device__ __forceinline__ float4 preview_shade(const JobDev& J, const HitT& h, 
 // 20,000 spherocylinders 2.8 -> 2.5, 500 meshes 6.4 -> 5.6, mixed 17.8 -> 16.2
 // against the 4 that 113 to 127 registers allow.
 template<int BLOCK, int SS, uint32_t TYPES, bool SPLIT>
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_preview(const JobDev* __restrict__ jobp, uint32_t aa_n,
-                                                   uint32_t own_search, uint2* gstack, uint32_t gstride,
-                                                   unsigned long long* counters)
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(6))) void k_preview(
+    const JobDev* __restrict__ jobp, uint32_t aa_n, uint32_t own_search, uint2* gstack, uint32_t gstride,
+    unsigned long long* counters)
     {
     constexpr uint32_t WAVES = BLOCK / 64;
     static_assert(BLOCK == 256, "one thread per pixel and channel of a chunk");
@@ -2660,8 +2665,8 @@ __global__ void k_debug_trace(const SceneDev sc, const float* rays, uint32_t n, 
     LocalStack st;
     uint32_t dummy = 0, err = 0;
     HitT h;
-    trace_closest<LocalStack, false, TYPES, true>(sc, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), tnear, h, st, dummy, dummy,
-                                     err);
+    trace_closest<LocalStack, false, TYPES, true>(sc, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), tnear, h, st,
+                                                  dummy, dummy, err);
     hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, err);
     }
     } // namespace fh

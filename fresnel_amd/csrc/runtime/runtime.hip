@@ -433,8 +433,8 @@ static void launch_traverse(DeviceObj& D, const char* nm, hipStream_t s, const T
              [&]
              {
                  kern<<<grid, TRAV_BLOCK, 0, s>>>(a.jobs, a.n_jobs, a.q, a.n, a.view, a.hits, a.work, a.chunk,
-                                                 D.xcd_bands == 2 ? 1u : 0u, std::min<uint32_t>(D.trav_refill, 64), a.gstack, a.gstride,
-                                                 a.counters);
+                                                 D.xcd_bands == 2 ? 1u : 0u, std::min<uint32_t>(D.trav_refill, 64),
+                                                 a.gstack, a.gstride, a.counters);
              });
     }
 
@@ -1900,6 +1900,10 @@ struct BatchExec
     // 256, 8 samples, whose few rays leave the separate kernels idle longer,
     // spherocylinders at 3.9, 16 and 63 0.26 / 0.38, 0.44 / 0.46, 0.70 / 0.56,
     // triangles at 13, 50 and 200 0.33 / 0.37, 0.47 / 0.45, 0.86 / 0.58.
+    // The line at 4 primitives per 64 pixels (from 4 Mi rays on) lies between
+    // the triangles' 2 and 8; spherocylinders would gain from 2.5 on.  The
+    // primitives are those of the whole scene over the whole image, in view or
+    // not.
     // Spheres stay with packets (their test is the cheapest: 1.56 / 1.62 at
     // 78), as do tile lists, and scenes with polyhedra, whose hits below their
     // bound (CULL_K) depend on the search's order.

@@ -312,8 +312,9 @@ int fh_policy_simulate(uint32_t n, const uint64_t* footprint, const uint64_t* pa
 
 /* ------------------------------------------------------ tuning (no reference
  * counterpart).  key "batch_paths": light-sample paths per wavefront batch
- * (default 256 Mi; sizes the ray queues, ≈ 160 B per path per render scratch); "tail_rays": below this many live
- * rays a batch finishes its paths in one kernel (default 524288); "stack_lds":
+ * (default 256 Mi; sizes the ray queues, ≈ 160 B per path per render scratch);
+ * "tail_rays": below this many live rays a batch finishes its paths in one
+ * kernel (default 524288); "stack_lds":
  * traversal stack entries kept in LDS per thread, 8 or 16 (default 8);
  * "trav_chunk": rays a secondary-ray traversal wavefront claims per
  * work-counter atomic, a multiple of 64 up to 65536 (default 256; fewer when
@@ -322,8 +323,9 @@ int fh_policy_simulate(uint32_t n, const uint64_t* footprint, const uint64_t* pa
  * once, a multiple of 64 up to 65536 (default 1024; a batch with fewer than 16
  * such claims per CU claims less, down to 256); "trav_refill": a traversal lane
  * whose ray is done takes a new one once this many lanes of its wavefront are
- * idle, 1..64 (65 counts as 64: all lanes; default 32); "trav_packet": primary rays traced as wavefront
- * packets (2, default) or one by one (1); "primary_tiles": primary rays of
+ * idle, 1..64 (65 counts as 64: all lanes; default 32); "trav_packet": primary
+ * rays traced as wavefront packets (2, default) or one by one (1);
+ * "primary_tiles": primary rays of
  * pinhole-perspective and orthographic cameras tested against per-8x8-tile
  * candidate lists (2, default) or searched in the BVH (1); "tile_min_rays":
  * with lists on, a tracer builds them once this many primary rays have been
@@ -338,8 +340,8 @@ int fh_policy_simulate(uint32_t n, const uint64_t* footprint, const uint64_t* pa
  * take as 2); "fuse_primary":
  * primary traversal and depth-0 shading in one kernel (2, default) or two (1);
  * "fuse_bounce": the same for each bounce of the secondary rays (default 1:
- * the fused kernel holds 88 registers, and the latency-bound secondary
- * traversal runs faster at the 8 wavefronts per SIMD of the separate kernel);
+ * the separate traversal refills its lanes and runs at 7 wavefronts per SIMD in
+ * spheres-only scenes, 6 in others);
  * "inflight": batches of one render kept in flight on the device's two
  * render streams (2, default: one batch's kernels run while the host waits
  * for the other's queue counts) or 1; "xcd_bands": the primary kernel fills

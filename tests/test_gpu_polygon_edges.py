@@ -44,7 +44,7 @@ def build(device, vertices, rounding):
 @pytest.mark.parametrize('rounding', [0.0, 0.1])
 @pytest.mark.parametrize('name', sorted(POLYGONS))
 def test_polygon_edges_equal_checker(name, rounding, gpu_device, cpu_device):
-    """Rays at vertices, edge midpoints, points on edges and their neighbours; an image with outlines (edge distances)."""
+    """Rays at vertices, edge midpoints, points on edges and their neighbours; an image with outlines."""
     v = numpy.array(POLYGONS[name], dtype=numpy.float32)
     gs, cs = build(gpu_device, v, rounding), build(cpu_device, v, rounding)
     rng = numpy.random.default_rng(9)
@@ -55,10 +55,11 @@ def test_polygon_edges_equal_checker(name, rounding, gpu_device, cpu_device):
     p = p.astype(numpy.float32)
     p = numpy.concatenate([p, numpy.nextafter(p, numpy.float32(9)), numpy.nextafter(p, numpy.float32(-9))])
     down = numpy.tile(numpy.float32([0, 0, -1]), (len(p), 1))
-    rays = [numpy.concatenate([p, numpy.ones((len(p), 1)), down], axis=1)]
+    height = numpy.ones((len(p), 1))
+    rays = [numpy.concatenate([p, height, down], axis=1)]
     tilted = rng.normal(size=(len(p), 3)) * [0.3, 0.3, 0] + [0, 0, -1]
     tilted /= numpy.linalg.norm(tilted, axis=1, keepdims=True)
-    rays.append(numpy.concatenate([p - tilted[:, :2] / tilted[:, 2:], numpy.full((len(p), 1), 0.0) + 1, tilted], axis=1))
+    rays.append(numpy.concatenate([p + tilted[:, :2] / tilted[:, 2:], height, tilted], axis=1))
     rays = numpy.ascontiguousarray(numpy.concatenate(rays), dtype=numpy.float32)
     n = len(rays)
     gid, prim, t = gs._scene.debugTrace(rays, 1e-3)

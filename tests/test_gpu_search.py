@@ -1,4 +1,4 @@
-"""The 4-wide search against brute force: directions with zero and tiny components, flat and tiny scenes, few primitives."""
+"""The 4-wide search against brute force: zero and tiny direction components, flat, tiny and huge scenes."""
 
 import ctypes
 
