@@ -404,12 +404,13 @@ def run_plain(args):
     ctr = d.countersLast()
     d.countersEnable(False)
     pb = wl['prim_bytes']
-    traffic, valu_busy, valu_lanes = {}, {}, {}
+    traffic, traffic_rays, valu_busy, valu_lanes = {}, {}, {}, {}
     tf = os.path.join(ROOT, 'profiles', f'traffic_{args.workload}.json')
     if os.path.exists(tf):
         with open(tf) as f:
             prof = json.load(f)
         traffic = prof.get('hbm_bytes_per_launch', {})
+        traffic_rays = prof.get('rays_per_launch', {})
         valu_busy = prof.get('valu_busy_pct', {})
         valu_lanes = prof.get('valu_active_lanes_pct', {})
 
@@ -430,6 +431,9 @@ def run_plain(args):
         flops = flops_node * nodes + FLOPS_PER_SPHERE * prims + FLOPS_PER_RAY * rays
         tflops = flops / (ms / 1e3) / 1e12 if ms > 0 else 0.0
         t = traffic.get(name)
+        if t and traffic_rays.get(name):
+            # the profile's launches may hold another number of rays than these
+            t = int(t * (rays / launches) / traffic_rays[name])
         measured_gbs = (t / (ms / launches / 1e3) / 1e9) if (t and ms > 0) else None
         busy = valu_busy.get(name)
         lanes = valu_lanes.get(name)
