@@ -2665,8 +2665,12 @@ __global__ void k_debug_trace(const SceneDev sc, const float* rays, uint32_t n, 
     LocalStack st;
     uint32_t dummy = 0, err = 0;
     HitT h;
-    trace_closest<LocalStack, false, TYPES, true>(sc, mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), tnear, h, st,
-                                                  dummy, dummy, err);
+    const v3 o = mk3(r[0], r[1], r[2]), d = mk3(r[3], r[4], r[5]);
+    // the 4-wide search takes boxes behind the origin as closed
+    if (tnear < 0.0f)
+        trace_binary<LocalStack, false, TYPES>(sc, o, d, tnear, h, st, dummy, dummy, err);
+    else
+        trace_closest<LocalStack, false, TYPES, true>(sc, o, d, tnear, h, st, dummy, dummy, err);
     hits[i] = make_uint4(__float_as_uint(h.t), h.geom, h.prim, err);
     }
     } // namespace fh

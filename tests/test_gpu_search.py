@@ -74,8 +74,8 @@ def rays_of(scene, n, rng):
     return numpy.ascontiguousarray(numpy.concatenate([o, d], axis=1), dtype=numpy.float32)
 
 
-@pytest.mark.parametrize('tnear', [0.0, 1e-3])
-@pytest.mark.parametrize('name', sorted(SCENES))
+@pytest.mark.parametrize('name,tnear', [(name, tnear) for name in sorted(SCENES) for tnear in (0.0, 1e-3)]
+                         + [(name, -3.0) for name in ('spheres_1', 'spheres_5', 'flat', 'box', 'cylinders', 'polygons')])
 def test_search_equals_brute_force(name, tnear, gpu_device, cpu_device):
     """Geometry, primitive and distance of every ray are the brute-force minimum's, bit for bit."""
     gs, cs = SCENES[name](gpu_device), SCENES[name](cpu_device)
