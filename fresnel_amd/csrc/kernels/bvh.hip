@@ -526,8 +526,9 @@ __device__ __forceinline__ void child_box(const Node& n, uint32_t side, float b[
 // An end that is infinite, NaN or beyond 2^66 becomes -2^66 (a low end) or 2^66
 // (a high one), the largest interval whose slab test cannot overflow (2^67
 // times RCP_MAX, 2^60), above the 2^64 at which squared distances overflow in
-// the primitives' own tests.  A primitive's own bounds are tested exactly at
-// its leaf, so one out there is still found by every ray that starts within.
+// the primitives' own tests; only that axis takes their pad.  A primitive's own
+// bounds are tested exactly at its leaf, so one out there is still found by
+// every ray that starts within.
 __global__ void k_bvh4_fill(const Node* __restrict__ nodes, uint32_t n, const uint32_t* __restrict__ idx4,
                             const uint32_t* __restrict__ parent, Node4* __restrict__ out)
     {
@@ -582,26 +583,47 @@ __global__ void k_bvh4_fill(const Node* __restrict__ nodes, uint32_t n, const ui
         ref[1] = ref[0];
         m = 2;
         }
+    // a box of NaN alone (primitives of NaN positions, and nodes of nothing
+    // else) lets no ray pass its slab test: that child is closed, high below low
     constexpr float FAR = 0x1p66f;
+    bool closed[4];
+    bool far[3] = {false, false, false};
     float big = 0.0f;
     for (uint32_t k = 0; k < m; k++)
+        {
+        closed[k] = true;
         for (int x = 0; x < 6; x++)
+            closed[k] = closed[k] && box[k][x] != box[k][x];
+        for (int x = 0; x < 6 && !closed[k]; x++)
             {
-            if (!(fabsf(box[k][x]) <= FAR))
+            if (fabsf(box[k][x]) <= FAR)
+                big = fmaxf(big, fabsf(box[k][x]));
+            else
+                {
                 box[k][x] = (x < 3) ? -FAR : FAR;
-            big = fmaxf(big, fabsf(box[k][x]));
+                far[x % 3] = true;
+                }
             }
-    const double pad = (double)NODE_PAD * big;
+        }
     Node4 r;
     for (int x = 0; x < 3; x++)
         {
         // swapped ends (a negative radius) count as the interval between them
         double lo = 1e300, hi = -1e300;
         for (uint32_t k = 0; k < m; k++)
+            if (!closed[k])
+                {
+                lo = fmin(lo, (double)fminf(box[k][x], box[k][3 + x]));
+                hi = fmax(hi, (double)fmaxf(box[k][x], box[k][3 + x]));
+                }
+        if (!(lo <= hi))
             {
-            lo = fmin(lo, (double)fminf(box[k][x], box[k][3 + x]));
-            hi = fmax(hi, (double)fmaxf(box[k][x], box[k][3 + x]));
+            // every child closed: ends as far apart as can be
+            lo = -(double)FAR;
+            hi = (double)FAR;
+            far[x] = true;
             }
+        const double pad = (double)NODE_PAD * (far[x] ? FAR : big);
         // one step of head room on each side: origin and step are rounded to float
         const float step = (float)((hi - lo + 2.0 * pad) * (1.0 / 253.0)) + 0x1p-126f;
         const float org = (float)(lo - pad - (double)step);
@@ -610,7 +632,8 @@ __global__ void k_bvh4_fill(const Node* __restrict__ nodes, uint32_t n, const ui
             {
             const double a = (double)fminf(box[k][x], box[k][3 + x]) - pad - (double)org;
             const double b = (double)fmaxf(box[k][x], box[k][3 + x]) + pad - (double)org;
-            const double fa = floor(a / (double)step), fb = ceil(b / (double)step);
+            const double fa = closed[k] ? 255.0 : floor(a / (double)step);
+            const double fb = closed[k] ? 0.0 : ceil(b / (double)step);
             ql |= (uint32_t)fmin(fmax(fa, 0.0), 255.0) << (8 * k);
             qh |= (uint32_t)fmin(fmax(fb, 0.0), 255.0) << (8 * k);
             }
