@@ -431,9 +431,10 @@ __device__ inline void trace_binary(const SceneDev& sc, v3 o, v3 d, float tnear,
 //   * the exact slab gate of a primitive's own bounds and its intersector run
 //     at the leaf step.  Leaf children are sorted and pushed like inner ones;
 //     a lane that takes one waits until enough lanes hold one.
-// A child is culled when its key, max(tmin, 0) - CULL_K tmax, exceeds the
-// closest hit plus the scene's margin (cull_bound with the margin moved to
-// the other side; CULL_K's factor of two covers the roundings of key and sum).
+// A child is culled when its key, max(tmin, 0 or tnear) - CULL_K tmax, exceeds
+// the closest hit plus the scene's margin (cull_bound with the margin moved to
+// the other side; CULL_K's factor of two covers the roundings of key and sum;
+// a hit lies past tnear, so the larger of the two bounds holds).
 // So every primitive whose bounds pass the slab test and whose hit does not lie
 // below its own culling bound is tested if it could still win, and the result
 // is the smallest (t, geometry, primitive) of those whatever the hierarchy and
@@ -553,12 +554,14 @@ __device__ __forceinline__ void order2(float& ka, uint32_t& na, float& kb, uint3
     }
 
 // One node visit: the nearest open child is taken next, the others are pushed,
-// farthest first.  The near distance is held at 0, not at tnear, so a ray that
-// leaves a surface opens the padded boxes it starts in: in flat systems that
-// costs visits (polygons: 8.3 a secondary ray, the binary tree with its exact
-// boxes and tnear 1.0), with tnear in its place 10,000 hexagons took 4 % less
-// a call and 4,096 spheres 2 % more.
-template<class Stack, bool COUNT>
+// farthest first.  The near distance is held at tnear, which a primitive's own
+// gate asks its far end to reach, so a ray that leaves a surface does not open
+// the boxes it only starts in: in flat systems those are most of them (20,000
+// overlapping polygons, 800 x 600, 16 samples: at 0 in place of tnear 89 visits
+// a secondary ray and 14.7 ms a call, so 1.0 and 8.6; 10,000 hexagons 2.70 and
+// 2.59 ms).  Spheres-only kernels keep 0: their rays' origins lie in few boxes,
+// and 4,096 spheres took 2 % more with tnear.
+template<class Stack, bool COUNT, uint32_t TYPES>
 __device__ __forceinline__ void search_visit(const Node4* __restrict__ nodes, Search& r, Stack& st, uint32_t& n_nodes,
                                              uint32_t& err)
     {
@@ -584,7 +587,7 @@ __device__ __forceinline__ void search_visit(const Node4* __restrict__ nodes, Se
         const float tx = __builtin_fmaf(byte(qnx), sx, bx), ux = __builtin_fmaf(byte(qfx), sx, bx);
         const float ty = __builtin_fmaf(byte(qny), sy, by), uy = __builtin_fmaf(byte(qfy), sy, by);
         const float tz = __builtin_fmaf(byte(qnz), sz, bz), uz = __builtin_fmaf(byte(qfz), sz, bz);
-        const float lo = fmaxf(fmaxf(fmaxf(tx, ty), tz), 0.0f);
+        const float lo = fmaxf(fmaxf(fmaxf(tx, ty), tz), TYPES == T_SPHERES ? 0.0f : r.tnear);
         const float hi = fminf(fminf(ux, uy), uz) * (1.0f + 0x1p-19f);
         const float q = __builtin_fmaf(-CULL_K, hi, lo);
         const bool open = (lo <= hi) & !(q > r.cull) & (k < 2 || nd[k] != EMPTY);
@@ -730,7 +733,7 @@ __device__ inline void trace_closest(const SceneDev& scene, v3 o, v3 d, float tn
             if (n_in == 0 || n_leaf >= LEAF_WAIT * n_in)
                 break;
             if (inner)
-                search_visit<Stack, COUNT>(sc.nodes4(), r, st, n_nodes, err);
+                search_visit<Stack, COUNT, TYPES>(sc.nodes4(), r, st, n_nodes, err);
             }
         const bool leaf = (r.cur & LEAF) && r.cur != EMPTY;
         if (__ballot(leaf) == 0)
@@ -1309,7 +1312,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(TYPES == 
             if (n_in == 0 || n_leaf >= LEAF_WAIT * n_in || (more && n_in + n_leaf + refill <= 64))
                 break;
             if (inner)
-                search_visit<LdsStack<SS>, COUNT>(sc.nodes4(), r, st, n_nodes, err);
+                search_visit<LdsStack<SS>, COUNT, TYPES>(sc.nodes4(), r, st, n_nodes, err);
             }
         if (n_leaf != 0 && n_leaf >= LEAF_WAIT * n_in)
             if ((r.cur & LEAF) && r.cur != EMPTY)

@@ -182,3 +182,23 @@ def test_nan_positions(kind, axes, gpu_device):
     numpy.testing.assert_array_equal(images[1], images[0])
     # (at x alone NaN the visits of the exact binary search grow by a factor of 2.4 here)
     assert visits[1] < (1.01 if axes == slice(0, 3) else 4) * visits[0]
+
+
+def test_flat_scene_visits(gpu_device):
+    """Secondary rays that leave overlapping polygons in one plane do not walk the boxes they start in."""
+    d = gpu_device._device
+    rng = numpy.random.default_rng(3)
+    s = fresnel.Scene(gpu_device, lights=fresnel.light.cloudy())
+    fresnel.geometry.Polygon(s, [[-0.3, -0.3], [0.3, -0.3], [0, 0.3]], position=rng.uniform(-4, 4, (5000, 2)),
+                             angle=rng.uniform(0, 6, 5000), color=(0.4, 0.5, 0.6))
+    s.camera = fresnel.camera.Orthographic(position=(0, 0, 5), look_at=(0, 0, 0), up=(0, 1, 0), height=8)
+    t = fresnel.tracer.Path(gpu_device, w=160, h=120)
+    d.countersEnable(True)
+    try:
+        t.sample(s, samples=4)
+        c = d.countersLast()
+    finally:
+        d.countersEnable(False)
+    assert c[0] + c[6] > 10000
+    # 1.0 with exact boxes: the root, whose children a ray leaves before tnear unless it grazes the plane
+    assert (c[1] + c[7]) / (c[0] + c[6]) < 4
