@@ -421,13 +421,13 @@ __device__ inline void trace_binary(const SceneDev& sc, v3 o, v3 d, float tnear,
 // are tested later, many lanes together:
 //   * a child box is 8-bit steps of the node's interval (k_bvh4_fill); the
 //     ray's direction signs pick the near and far ends, so an axis of a
-//     child's slab interval is two byte conversions and two fmas.  The
-//     rounding of these (the node's origin less the ray's, exact operands, is
-//     one rounding) and of a primitive's float slab interval (lo - o) * inv
-//     is at most 5 x 2^-24 of the interval's end and 6 x 2^-24 of the node's
-//     largest coordinate times the reciprocal; the node's pad (2^-20 of that
-//     coordinate) and the factor 1 + 2^-19 in the comparison cover them, so
-//     every child whose primitives' own test could pass is open;
+//     child's slab interval is two byte conversions and two fmas.  The node's
+//     origin less the ray's is one rounding of exact operands, so an end at
+//     distance t is off by at most 3 x 2^-24 t, 3 x 2^-24 of the node's width
+//     times the reciprocal, and the 2 x 2^-24 t of a primitive's float slab
+//     interval (lo - o) * inv; the node's pad (2^-22 of its width and more)
+//     and the factor 1 + 2^-19 in the comparison cover them, so every child
+//     whose primitives' own test could pass is open;
 //   * the exact slab gate of a primitive's own bounds and its intersector run
 //     at the leaf step.  Leaf children are sorted and pushed like inner ones;
 //     a lane that takes one waits until enough lanes hold one.
@@ -488,8 +488,8 @@ struct Search
 
 // Reciprocal of a direction component for the node tests.  Below 2^-60 it is
 // taken as 2^60: a box the origin lies beside by more than the node's pad is
-// missed, and inside one the interval reaches 2^40 times the node's largest
-// coordinate, past every hit.
+// missed, and inside one the interval reaches 2^60 times that pad, at least
+// 2^36 times the node's largest coordinate, past every hit.
 constexpr float RCP_MAX = 0x1p60f;
 __device__ __forceinline__ float node_rcp(float d)
     {

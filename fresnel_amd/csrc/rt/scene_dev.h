@@ -93,7 +93,7 @@ struct __attribute__((aligned(64))) Node4
     uint32_t qlo[3], qhi[3];
     uint32_t ref[4];
     };
-constexpr float NODE_PAD = 0x1p-20f;
+constexpr double NODE_PAD = 0x1p-22, NODE_PAD_FLOOR = 0x1p-24;
 
 struct SceneDev
     {

@@ -202,3 +202,33 @@ def test_flat_scene_visits(gpu_device):
     assert c[0] + c[6] > 10000
     # 1.0 with exact boxes: the root, whose children a ray leaves before tnear unless it grazes the plane
     assert (c[1] + c[7]) / (c[0] + c[6]) < 4
+
+
+@pytest.mark.parametrize('kind', ['spheres', 'cylinders'])
+def test_far_from_the_origin_visits(kind, gpu_device):
+    """A scene moved by 2^20 (coordinates in steps of 1/8, exact in both places): about the same node visits."""
+    d = gpu_device._device
+    visits = []
+    for offset in (0, 2**20):
+        rng = numpy.random.default_rng(3)
+        pos = rng.integers(-120, 120, (20000, 3)) / 8.0 + offset
+        s = fresnel.Scene(gpu_device, lights=fresnel.light.cloudy())
+        m = fresnel.material.Material(color=(0.3, 0.5, 0.9), roughness=0.5)
+        if kind == 'spheres':
+            fresnel.geometry.Sphere(s, position=pos, radius=0.5, material=m)
+        else:
+            end = pos + rng.integers(-8, 8, pos.shape) / 8.0
+            fresnel.geometry.Cylinder(s, points=numpy.stack([pos, end], axis=1), radius=0.125, material=m)
+        s.camera = fresnel.camera.Orthographic(position=(offset, offset, offset + 64), look_at=(offset, offset, offset),
+                                               up=(0, 1, 0), height=32)
+        t = fresnel.tracer.Path(gpu_device, w=160, h=120)
+        t.seed = 2
+        d.countersEnable(True)
+        try:
+            t.sample(s, samples=4)
+            c = d.countersLast()
+        finally:
+            d.countersEnable(False)
+        visits.append((c[1] + c[7]) / (c[0] + c[6]))
+    # (the rays' own coordinates are steps of 1/8 there, so the paths differ)
+    assert visits[1] < 1.5 * visits[0]
