@@ -1162,6 +1162,16 @@ static void sync_scene(SceneObj& sc)
     if (sc.build_pending)
         HIPCHECK(hipStreamSynchronize(D.stream));
     sc.build_pending = false;
+    // an error below leaves copies that read host buffers: they end first
+    struct UploadsEnd
+        {
+        DeviceObj& D;
+        ~UploadsEnd()
+            {
+            if (D.uploads_queued)
+                (void)hipStreamSynchronize(D.copy_stream);
+            }
+        } uploads_end {D};
     bool any_dirty = false;
     std::vector<uint32_t> topo;
     for (auto& kv : sc.geoms)
@@ -1217,14 +1227,8 @@ static void sync_scene(SceneObj& sc)
         D.uploads_queued = true;
         HIPCHECK(hipMemcpyAsync(sc.dgeoms.p, table.data(), n_slots * sizeof(GeomDev), hipMemcpyHostToDevice,
                                 D.copy_stream));
+        sc.table = std::move(table); // (the rows the copy reads move along)
         }
-    // before the table and the colour buffers change and before the device
-    // stream's kernels read them; a colour edit uploads rows without a new
-    // table or hierarchy
-    if (D.uploads_queued)
-        uploads_done(D);
-    if (changed)
-        sc.table = std::move(table);
     sc.n_slots = n_slots;
     const bool topo_same = sc.bvh_valid && topo == sc.topo;
     if (!sc.bvh_valid || !topo_same)
@@ -1239,6 +1243,11 @@ static void sync_scene(SceneObj& sc)
         update_bvh(sc);
         sc.build_pending = true;
         }
+    // builds have waited for the uploads before their kernels; colour rows and
+    // the geometry table also change without one, and are waited for before
+    // they change again and before the device stream's kernels read them
+    if (D.uploads_queued)
+        uploads_done(D);
     sc.topo = topo;
     }
 
